@@ -45,6 +45,43 @@ def test_ctc_builder_matches_host_generator(seed):
     assert (fsa[1][3, edges.shape[1]:] == -1).all() and fsa[0] >= n_states
 
 
+# B * Lmax on both sides of FSA_SELF_COUNT (8192: the workgroups count earlier labels themselves, or a kernel in front
+# does), more labels than a workgroup has threads (1024), and sequences without labels
+@pytest.mark.parametrize("B,Lmax", [(1, 1), (3, 1100), (8, 1024), (9, 1024), (300, 2), (1500, 12)])
+def test_ctc_builder_sizes(B, Lmax):
+    from i6_native_ops_amd.fsa import ctc_fsa
+    rng = np.random.default_rng(B * 7 + Lmax)
+    lab, lens = ragged(rng, B, Lmax, 1, 4)
+    lens[-1] = Lmax
+    fsa, totals = ctc_fsa(torch.from_numpy(lab).to(DEV), torch.from_numpy(lens).to(DEV), blank=0, return_totals=True)
+    n_states, edges, weights, start_end = trimmed(fsa, totals)
+    want = _assemble("x", [_ctc(lab[b, :lens[b]].tolist(), blank=0) for b in range(B)], np.ones(B), 1, B, 4, rng, 1.0, False, False)
+    assert n_states == want.n_states
+    np.testing.assert_array_equal(edges, want.edges)
+    np.testing.assert_array_equal(start_end, want.start_end_states)
+    assert (weights == 0).all() and (fsa[1][3, edges.shape[1]:] == -1).all()
+
+
+@pytest.mark.parametrize("B,Lmax", [(1, 1), (2, 400), (1100, 3)])
+def test_hmm_builder_sizes(B, Lmax):
+    from i6_native_ops_amd.fsa import hmm_fsa
+    rng = np.random.default_rng(B * 5 + Lmax)
+    lab, lens = ragged(rng, B, Lmax, 0, 20)
+    lens[-1] = Lmax
+    lens[0] = max(1, lens[0])
+    fsa, totals = hmm_fsa(torch.from_numpy(lab).to(DEV), torch.from_numpy(lens).to(DEV), 3, 0.25, 1.5, return_totals=True)
+    n_states, edges, weights, start_end = trimmed(fsa, totals)
+    n = lens.astype(np.int64) * 3
+    first = np.concatenate([[0], np.cumsum(n + 1)])[:B]
+    np.testing.assert_array_equal(start_end, np.stack([first, first + n]))
+    assert n_states == int((n + 1).sum()) and edges.shape[1] == 2 * int(n.sum())
+    src = np.concatenate([first[b] + np.arange(n[b]) for b in range(B)])
+    emis = np.concatenate([np.repeat(lab[b, :lens[b]] * 3, 3) + np.tile(np.arange(3), lens[b]) for b in range(B)])
+    np.testing.assert_array_equal(edges[:, 0::2], np.stack([src, src, emis, np.repeat(np.arange(B), n)]))
+    np.testing.assert_array_equal(edges[:, 1::2], np.stack([src, src + 1, emis, np.repeat(np.arange(B), n)]))
+    np.testing.assert_array_equal(weights, np.tile(np.array([0.25, 1.5], np.float32), int(n.sum())))
+
+
 def test_ctc_loss_equals_torch(oracle):
     """fbw_loss over the built automaton (used at full capacity, padding edges included) against
     torch's CTC loss and its gradient on the CPU."""
