@@ -109,6 +109,11 @@ constexpr float LOG2E = 1.44269504088896341f;
 constexpr float LN2 = 0.693147180559945309f;
 #define INF_F __builtin_inff()
 
+// Strips of states (strip_kernels.inc): lanes of a wave that repeat the last states of the strip before (the first ones of
+// the strip behind, walking backward), states a strip advances by, largest number of strips of one sequence
+constexpr int STRIP_HALO = 4, STRIP_USE = 64 - STRIP_HALO, STRIP_MAX = (S_MAX + STRIP_HALO + STRIP_USE - 1) / STRIP_USE;
+constexpr int STRIP_FRAMES = 8;       // frames per block of the strip kernels
+
 struct SeqMeta {
     int edge_begin;   // edges with a smaller sequence index
     int n_edges;
@@ -120,7 +125,7 @@ struct SeqMeta {
     int err;          // common problems (written by the emission-order role)
     int Kin, errA;    // written by the target-order role
     int Kout, errB;   // written by the source-order role
-    int pad;          // bit 0: edges contiguous in the input
+    int pad;          // bit 0: edges contiguous in the input; bit 1: states renumbered; bit 2: their numbers stand in a plain array; bits 8 and up: see live_window
 };
 
 __host__ __device__ inline long long round16(long long x) { return (x + 15) & ~15LL; }
@@ -128,6 +133,8 @@ __host__ __device__ inline long long round16(long long x) { return (x + 15) & ~1
 // prefix sum over sequences (and no cross-workgroup dependency) is needed.
 __host__ __device__ inline long long state_off(long long edge_begin, int b) { return round16(2 * edge_begin) + 32LL * b; }
 __host__ __device__ inline long long slot_off(long long edge_begin, int b) { return round16(edge_begin) + 32LL * b; }
+// (floats per frame of the strip kernels' score table, see strip_kernels.inc)
+__host__ __device__ inline long long strip_off(long long edge_begin, int b) { return round16(edge_begin + (edge_begin >> 1) + (edge_begin >> 2)) + 272LL * b; }
 // Entries of a sequence's renumbering table (see local_state) and the home position of a state id in it
 __host__ __device__ inline unsigned renum_capacity(int n_edges) { return 2u * (2u * (unsigned)n_edges + 16u); }
 __host__ __device__ inline unsigned renum_home(int id, unsigned cap) {
@@ -135,7 +142,7 @@ __host__ __device__ inline unsigned renum_home(int id, unsigned cap) {
 }
 
 struct Layout {
-    size_t meta, sync, sortflag, seqbegin, eidx, ellA, ellB, crec, cbegin, demis, tband, renum, cflag, wpfx, offA, offB, alpha, beta, gtab, total;
+    size_t meta, sync, sortflag, seqbegin, eidx, ellA, ellB, crec, cbegin, demis, tband, renum, cflag, wpfx, offA, offB, alpha, beta, gtab, base_total, sprog, etab, total;
     long long ss_total, gg_total;
     int wpfx_stride;      // ints per sequence in the emission rank table (0: F too large for it)
 };
@@ -168,6 +175,10 @@ Layout make_layout(long long T, long long B, long long E, long long F = 1) {
     // (behind everything else: the offsets above do not depend on F)
     l.cflag = o;    o = align256(o + sizeof(int) * B * ((T + FLAT_TCF - 1) / FLAT_TCF));
     l.wpfx = o;     o = align256(o + sizeof(int) * B * l.wpfx_stride);
+    l.base_total = o;
+    // (the strip kernels' share; a call whose workspace ends before it runs without them)
+    l.sprog = o;    o = align256(o + sizeof(int) * 2 * STRIP_MAX * B);
+    l.etab = o;     o = align256(o + sizeof(float) * (strip_off(E, (int)B) + 16) * (((size_t)T + 7) & ~(size_t)7));
     l.total = o;
     return l;
 }
@@ -208,6 +219,21 @@ __device__ inline int rec_class(const SeqMeta& m, const int threads = REC_THREAD
     if (m.SP <= threads && m.DP <= (threads > 512 ? 1024 : 512)) return 1;     // (the loader wave of the large instance takes rows of 1024)
     if (m.SP <= 4 * threads && m.DP <= 2048) return 2;
     return 3;
+}
+
+// Number of strips of a sequence that the strip kernels take (strip_kernels.inc), 0 for all others.  They need states
+// numbered so that no edge leads downward and none raises the number by more than the halo, edges that fit the registers,
+// and tables that fit the sequence's share of the workspace; `most` is what the host has launched waves for.
+__device__ inline int strip_count(const SeqMeta& m, const int b, const int T, const int most) {
+    const int d = m.pad >> 8;
+    if (d < 1 || d > STRIP_HALO || seq_error(m) != 0 || m.L == 0 || m.n_edges == 0 || m.Kin > KMAX || m.Kout > KMAX) return 0;
+    const int n = (m.S + STRIP_HALO + STRIP_USE - 1) / STRIP_USE;
+    if (n > most) return 0;
+    if (64LL * (d == 1 ? 2 : 3) * n > strip_off(m.edge_begin + m.n_edges, b + 1) - strip_off(m.edge_begin, b)) return 0;
+    // (alpha's area also holds back-pointers and halo values of the best-path search: 80 bytes per strip and frame)
+    const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
+    if (80LL * n * T8 > 4LL * T * (state_off(m.edge_begin + m.n_edges, b + 1) - state_off(m.edge_begin, b))) return 0;
+    return n;
 }
 
 // Hand-off between kernels that run at the same time (gather -> recursion -> combine).  The
@@ -305,6 +331,8 @@ struct PrepArgs {
     int* cflag = nullptr;   // per (sequence, strip of TC frames): compact posteriors written (flat dense write); may be null
     int* wpfx = nullptr;    // per sequence: number of distinct emissions below 32 * w, for w = 0 .. ceil(F / 32); may be null
     int wpfx_stride = 0;
+    int strips = 0;         // > 0: sequences of up to that many strips go to the strip kernels
+    int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence
 };
 
 // sortflag[blk] = 1 if the sequence indices of edges [blk*SCAN_BLOCK, (blk+1)*SCAN_BLOCK] never
@@ -427,7 +455,7 @@ __device__ __forceinline__ void bitonic_sort_in_registers(unsigned* keys, const 
     __syncthreads();
 }
 
-constexpr int PREP_AUX_WORDS = 2048;   // scratch words of a preparation workgroup beside its sort keys
+constexpr int PREP_AUX_WORDS = 2048;   // scratch words of a preparation workgroup beside its sort keys (two state numbers each)
 constexpr int KEY_POS_BITS = 13;   // EB_MAX = 2^13 positions; the primary key sits above them
 static_assert((1 << KEY_POS_BITS) == EB_MAX, "key layout");
 
@@ -550,12 +578,12 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
     // Sequences whose ids, spread or not, do not follow the automaton (some edge leads to a smaller id) get numbers along
     // the automaton where that matters (by_level below): that is what the recursion's renormalisation over live states
     // and the activity band of the gather go by (live_window, min_steps).
-    const bool unordered = !err && n_edges > 0 && s_nonmono != 0 && s_bad == 0 && n_edges <= RENUM_LDS_EDGES && !a.force_generic;
+    const bool unordered = !err && n_edges > 0 && s_nonmono != 0 && s_bad == 0 && n_edges <= EB_MAX && !a.force_generic;
     // ... and such a sequence is ranked too when its ids, without being spread by the measure above, span more than the
     // numbering below can hold, as the ids of one sequence among many do after a permutation over the whole batch (a chain
     // of 1020 states with ids out of 3573, 1100 frames: 7.9e-5 before): the span says nothing about the number of states then
     constexpr int LEVEL_STATES = EB_MAX / 4;
-    const bool span_too_wide = unordered && !sparse && S > LEVEL_STATES && L > 0 && 5LL * S > 4LL * L;
+    const bool span_too_wide = unordered && n_edges <= RENUM_LDS_EDGES && !sparse && S > LEVEL_STATES && L > 0 && 5LL * S > 4LL * L;
     bool ranked = (sparse || span_too_wide) && n_edges <= RENUM_LDS_EDGES && !a.force_generic;
     if (sparse && !ranked) generic = 1;
     if (n_edges == 0) S = 1;
@@ -627,37 +655,33 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
     };
     // Numbers along the automaton for a sequence whose ids do not follow it, where that matters: a tightly aligned one,
     // fewer than five frames for every four states (chains of 1021 states over 1021-1100 frames came out at 9.9e-5 under
-    // permuted ids; the long-form configuration, whose optional states carry the highest ids, is at 2.5e-5 with 1.6
-    // frames per state and would pay 0.17 ms per call).  A state's height is the length of the longest path from it,
+    // permuted ids).  A state's height is the length of the longest path from it,
     // self-loops aside, so every other edge leads to a lower state, and the states are numbered by falling height, then
     // by id.  Heights by policy iteration: every state picks the highest of its successors, the heights along the chosen
     // chains are added up by pointer jumping (log2 S rounds), and the states pick again, until every state sits exactly
     // one above its highest successor -- two or three picks for a chain with optional states, whatever the order of
     // ids and edges (one round per state, as relaxation needs, cost such a call a millisecond).  An automaton that has
     // not come to rest after LEVEL_PICKS picks (a cycle through several states never does) keeps the ranks of its ids, as
-    // does one with more than LEVEL_STATES states.  Every role arrives at the same numbers.
+    // does one with more states than fit (ranked ids take up half of the work space).  Every role arrives at the same numbers.
+    // Where the strip kernels are in use every sequence whose ids do not follow it gets them: they need states whose edges lead upward.
     constexpr int LEVEL_PICKS = 8;
-    static_assert(LEVEL_STATES <= PREP_AUX_WORDS && LEVEL_STATES <= 4096, "height << 16 | state; sort key height << 12 | state");
-    unsigned* dn = uniq + LEVEL_STATES;          // [S]: hops to the end of the chain of chosen successors << 16 | that end; later: the state's number
-    bool by_level = unordered && (ranked || !sparse) && !generic && S <= LEVEL_STATES && L > 0 && 5LL * S > 4LL * L;
+    static_assert(2 * PREP_AUX_WORDS >= S_MAX && S_MAX <= 4096 && EB_MAX >= 2 * S_MAX, "height << 16 | state; sort key height << 12 | state");
+    unsigned* dn = ranked ? uniq + LEVEL_STATES : uniq;     // [S]: hops to the end of the chain of chosen successors << 16 | that end
+    unsigned short* num = (unsigned short*)aux;              // [S]: the state's number
+    bool by_level = unordered && (ranked || !sparse) && !generic && S <= (ranked ? LEVEL_STATES : S_MAX) && L > 0 && (a.strips > 0 || 5LL * S > 4LL * L);
     if (by_level) {
-        unsigned* pk = keys;                      // the edges as ranks: source | target << 16
-        unsigned* cand = aux;                     // [S]: (height of the best successor + 1) << 16 | that successor
-        constexpr int SPT = LEVEL_STATES / NT;    // states per thread
+        unsigned* cand = keys;                    // [S]: (height of the best successor + 1) << 16 | that successor
+        constexpr int SPT = S_MAX / NT;           // states per thread
         const int nS = (int)S;
         __syncthreads();        // the edge list written above (an edge list that is not grouped by sequence is read through it)
-        for (int i = tid; i < n_edges; i += NT) {
-            const int e = edge_at(i);
-            pk[i] = rank_of((unsigned)e_from[e]) | (rank_of((unsigned)e_to[e]) << 16);
-        }
         for (int r = tid; r < nS; r += NT) dn[r] = (unsigned)r;
-        __syncthreads();
         bool rest = false;
         for (int pick = 0; pick < LEVEL_PICKS && !rest; pick++) {
             for (int r = tid; r < nS; r += NT) cand[r] = 0u;
             __syncthreads();
             for (int i = tid; i < n_edges; i += NT) {
-                const unsigned u = pk[i] & 0xFFFFu, w = pk[i] >> 16;
+                const int e = edge_at(i);
+                const unsigned u = rank_of((unsigned)e_from[e]), w = rank_of((unsigned)e_to[e]);
                 if (u != w) atomicMax(&cand[u], (((dn[w] >> 16) + 1u) << 16) | w);
             }
             __syncthreads();
@@ -672,6 +696,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
                 for (int j = 0; j < SPT; j++) {
                     const int r = tid + j * NT;
                     q[j] = 0u;
+                    if (j * NT >= nS) break;
                     if (r < nS) {
                         const unsigned a_ = dn[r], b_ = dn[a_ & 0xFFFFu];
                         q[j] = (min((a_ >> 16) + (b_ >> 16), 4095u) << 16) | (b_ & 0xFFFFu);      // (a cycle saturates and never comes to rest)
@@ -679,26 +704,31 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
                 }
                 __syncthreads();
 #pragma unroll
-                for (int j = 0; j < SPT; j++)
+                for (int j = 0; j < SPT; j++) {
+                    if (j * NT >= nS) break;
                     if (tid + j * NT < nS) dn[tid + j * NT] = q[j];
+                }
                 __syncthreads();
             }
         }
         if (!rest) by_level = false;
         else {
-            int N3 = 2;
+            int N3 = NT;
             while (N3 < nS) N3 <<= 1;
             for (int i = tid; i < N3; i += NT) keys[i] = i < nS ? ((4095u - (dn[i] >> 16)) << 12) | (unsigned)i : ~0u;
             __syncthreads();
-            lds_bitonic_sort<NT>(keys, N3);
-            for (int i = tid; i < nS; i += NT) dn[keys[i] & 0xFFFu] = (unsigned)i;
+            if (N3 == NT) bitonic_sort_in_registers<NT, 1>(keys, tid);
+            else if (N3 == 2 * NT) bitonic_sort_in_registers<NT, 2>(keys, tid);
+            else if (N3 == 4 * NT) bitonic_sort_in_registers<NT, 4>(keys, tid);
+            else bitonic_sort_in_registers<NT, 8>(keys, tid);
+            for (int i = tid; i < nS; i += NT) num[keys[i] & 0xFFFu] = (unsigned short)i;
             __syncthreads();
         }
     }
     // state id -> number within the sequence
     auto local = [&](const unsigned id) -> unsigned {
         const unsigned r = rank_of(id);
-        return by_level ? dn[r] : r;
+        return by_level ? num[r] : r;
     };
     int SP = (int)round16(S);
     if (!err && !generic && n_edges > 0) {
@@ -729,7 +759,13 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
     const int DP = (int)round16(D > 0 ? D : 1);
 
     int start_loc = (int)local(st_state), end_loc = (int)local(en_state);
-    if ((sparse || ranked || by_level) && role == 2) {
+    const bool plain_table = by_level && !ranked && !sparse;
+    if (plain_table && role == 2) {
+        // numbers by place of the id in its range (S <= 2 n + 2 <= the table's room)
+        int2* tab = a.renum + 2 * soff;
+        for (int i = tid; i < (int)S; i += NT) tab[i] = make_int2(0, (int)num[i]);
+    }
+    if ((sparse || ranked) && role == 2) {
         // The general path looks the numbers up in an open-addressing table {id + 1, number} (see
         // local_state), which is written for every sequence whose numbers are not simply the place of the
         // id in its range: the other two roles may still send it there.  Numbers: the ones from above,
@@ -787,6 +823,8 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
             int* cf = a.cflag + (size_t)b * ncf;
             for (int i = tid; i < ncf; i += NT) cf[i] = 0;
         }
+        if (a.strips > 0)
+            for (int i = tid; i < 2 * STRIP_MAX; i += NT) a.sprog[(size_t)b * 2 * STRIP_MAX + i] = 0;
         if (tid == 0) atomicMax(&a.sync[6], L);      // longest sequence of the batch (header cleared by the scan kernel)
     }
     if (role == 2 && tid == 0) {
@@ -797,7 +835,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         m->err = err ? err : (generic ? SEQ_GENERIC : 0);
         // bit 0: the edges of the sequence are contiguous in the input; bit 1: its states are renumbered;
         // bits 8 and up: see below
-        m->pad = (sorted ? 1 : 0) | ((sparse || ranked || by_level) ? 2 : 0);
+        m->pad = (sorted ? 1 : 0) | ((sparse || ranked || by_level) ? 2 : 0) | (plain_table ? 4 : 0);
     }
     if (err || generic || n_edges == 0) {
         if (tid == 0) {
@@ -974,8 +1012,8 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         }
         __syncthreads();
         int2* tb = a.tband + goff;
-        // (the best-path search reads every frame: values outside the band would have to be -inf there)
-        for (int d = tid; d < DP; d += NT) tb[d] = (a.best_path || a.no_band) ? make_int2(0, 1 << 30) : make_int2(s_tlo[d], s_thi[d]);
+        // (the best-path search without strips reads every frame)
+        for (int d = tid; d < DP; d += NT) tb[d] = ((a.best_path && a.strips == 0) || a.no_band) ? make_int2(0, 1 << 30) : make_int2(s_tlo[d], s_thi[d]);
     }
 }
 
@@ -1013,16 +1051,11 @@ struct GatherArgs {
     int* sync;
     float scale;      // log2(e) for -log scores, -log2(e) for log scores
     int ascending;    // strips in ascending order (one consumer walking forward) instead of from both ends inwards
+    float fill = INF_F;   // value outside the band: one that never contributes
 };
 
 template <bool SYNC>
-__global__ __launch_bounds__(256) void fbw_gather(GatherArgs a) {
-    int b, y;
-    strip_index(a.B, &b, &y);
-#ifdef I6_TRACE
-    trace_corun(3110);
-#endif
-    const SeqMeta m = a.meta[b];
+__device__ __forceinline__ void gather_rows(const GatherArgs& a, const SeqMeta& m, const int b, const int y) {
     if (rec_class(m) <= 0) return;
     const int n = (m.L + TG - 1) / TG;
     if (y >= n) return;
@@ -1040,12 +1073,12 @@ __global__ __launch_bounds__(256) void fbw_gather(GatherArgs a) {
         float v[TG];
 #pragma unroll
         for (int tt = 0; tt < TG; tt++) {
-            v[tt] = INF_F;
+            v[tt] = a.fill;
             if (tt < nt && t0 + tt >= band.x && t0 + tt <= band.y) v[tt] = __builtin_nontemporal_load(&am[(long long)(t0 + tt) * a.st_t + e]);   // read once: keep it out of the caches
         }
 #pragma unroll
         for (int tt = 0; tt < TG; tt++)
-            if (tt < nt) store_x<SYNC>(&g[(size_t)(t0 + tt) * m.DP + idx], v[tt] == INF_F ? INF_F : v[tt] * a.scale);
+            if (tt < nt) store_x<SYNC>(&g[(size_t)(t0 + tt) * m.DP + idx], v[tt] == a.fill ? a.fill : v[tt] * a.scale);
     }
     if (SYNC) {
         wait_stores();
@@ -1055,6 +1088,17 @@ __global__ __launch_bounds__(256) void fbw_gather(GatherArgs a) {
 #ifdef I6_TRACE
     if (threadIdx.x == 0) { atomicMax(&g_trace[1], wall_clock64()); atomicMin(&g_trace[0], wall_clock64()); if (b == 0) g_trace[512 + j] = wall_clock64(); }
 #endif
+}
+
+template <bool SYNC>
+__global__ __launch_bounds__(256) void fbw_gather(GatherArgs a) {
+    int b, y;
+    strip_index(a.B, &b, &y);
+#ifdef I6_TRACE
+    trace_corun(3110);
+#endif
+    const SeqMeta m = a.meta[b];
+    gather_rows<SYNC>(a, m, b, y);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -3532,8 +3576,8 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     if (B > 65535 || (T + TC - 1) / TC > 65535) return I6FBW_ERR_INVALID_ARGUMENT;   // grid limits
     const Layout l = make_layout(T, B, E, F);
     if (static_call) {
-        if (l.total > (size_t)I6FBW_STATIC_WORKSPACE_BYTES) return I6FBW_ERR_STATIC_WORKSPACE;
-    } else if (workspace_bytes < l.total) return I6FBW_ERR_WORKSPACE_TOO_SMALL;
+        if (l.base_total > (size_t)I6FBW_STATIC_WORKSPACE_BYTES) return I6FBW_ERR_STATIC_WORKSPACE;
+    } else if (workspace_bytes < l.base_total) return I6FBW_ERR_WORKSPACE_TOO_SMALL;
     // too many emission classes for the LDS bitmap of the preparation: every sequence takes the general path
     const bool f_too_large = F > F_BITMAP_MAX;
     // rows too long for the LDS image of the dense write go through it in tiles; so do rows of more
@@ -3956,7 +4000,8 @@ int i6fbw_dump_alignment(const void* workspace, int T, int B, int E, const int32
             if (e != hipSuccess) { g_last_hip_error = e; fclose(f); return I6FBW_ERR_LAUNCH; }
             if (m.pad & 2) {
                 // state ids spread over a wide range: their numbers within the sequence sit in an open-addressing table
-                renum.resize(renum_capacity(m.n_edges));
+                // (or, for ids that are not spread, in an array by place of the id in its range)
+                renum.resize((m.pad & 4) ? (size_t)m.S : (size_t)renum_capacity(m.n_edges));
                 e = hipMemcpy(renum.data(), (const char*)workspace + l.renum + sizeof(int2) * 2 * (size_t)soff, sizeof(int2) * renum.size(),
                               hipMemcpyDeviceToHost);
                 if (e != hipSuccess) { g_last_hip_error = e; fclose(f); return I6FBW_ERR_LAUNCH; }
@@ -3965,6 +4010,7 @@ int i6fbw_dump_alignment(const void* workspace, int T, int B, int E, const int32
         // number of state id sid within the sequence, -1 if the sequence does not name it
         auto local = [&](long long sid) -> long long {
             if (!(m.pad & 2)) { const long long loc = sid - m.state_min; return loc >= 0 && loc < m.S ? loc : -1; }
+            if (m.pad & 4) { const long long loc = sid - m.state_min; return loc >= 0 && loc < m.S ? renum[(size_t)loc].y : -1; }
             const unsigned cap = (unsigned)renum.size();
             unsigned h = renum_home((int)sid, cap);
             while (true) {
@@ -4049,5 +4095,6 @@ int i6fbw_profile_read(float* stage_ms) {
 
 }  // extern "C"
 
+#include "strip_kernels.inc"
 #include "viterbi_kernels.inc"
 #include "fsa_builders.inc"

@@ -1,0 +1,139 @@
+"""The strip kernels (automata whose edges lead from a state to itself or up to four numbers upward) against the oracle,
+at the sizes where they can go wrong: strips of 60 states, workgroups of four strips, blocks of eight frames, back-pointer
+windows of 64 states, and every kind of edge they take or leave to the other kernels."""
+import numpy as np
+import pytest
+import torch
+
+from i6_native_ops_amd import cabi
+from tests.test_viterbi_gpu import assert_identical, run_cabi_viterbi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def stage_after_stage():
+    cabi.set_overlap(0)
+    yield
+    cabi.set_overlap(-1)
+
+
+def automata(rng, sizes, F, kind, permute=False):
+    """Left-to-right automata of the given numbers of states.  kind: "chain" loops and steps; "optional" some states can be
+    passed over; "ctc" emission on the target state and several edges into the last state; "wide" edges of up to four
+    states upward, some of them twice; "far" one edge of five (not for the strips).  Weights are multiples of 1/2, so ties are common."""
+    frm, to, emis, seq, w = [], [], [], [], []
+    ends = []
+    off = 0
+    for b, n in enumerate(sizes):
+        state_emis = rng.integers(0, F, size=n)
+
+        def edge(u, v, e):
+            frm.append(off + u); to.append(off + v); emis.append(int(e)); seq.append(b)
+            w.append(-0.5 * int(rng.integers(0, 4)))
+
+        for u in range(n):
+            by_target = kind in ("ctc", "wide")
+            steps = [0, 1]
+            if kind in ("optional", "ctc") and rng.random() < 0.4:
+                steps.append(2)
+            if kind == "wide":
+                steps += [int(x) for x in rng.integers(1, 5, size=rng.integers(0, 2))]
+            if kind == "far" and u == n // 3:
+                steps.append(5)
+            for k in steps:
+                if u + k < n and not (kind == "ctc" and u + k == n - 1 and k == 0):
+                    edge(u, u + k, state_emis[u + k] if by_target else state_emis[u])
+        if kind == "ctc" and n >= 5:
+            for u, v in ((n - 2, n - 2), (n - 3, n - 2), (n - 4, n - 2), (n - 2, n - 3)):
+                edge(u, n - 1, state_emis[v])
+        ends.append(off + n - 1)
+        off += n
+    starts = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    edges = np.array([frm, to, emis, seq], dtype=np.int32)
+    start_end = np.array([starts, ends], dtype=np.int32)
+    if permute:
+        # ids that do not follow the automaton, each sequence within its own range
+        new = np.concatenate([s + rng.permutation(n) for s, n in zip(starts, sizes)]).astype(np.int32)
+        edges[:2] = new[edges[:2]]
+        start_end = new[start_end].astype(np.int32)
+    order = rng.permutation(edges.shape[1])
+    return edges[:, order].copy(), np.array(w, dtype=np.float32)[order].copy(), start_end, off
+
+
+CASES = [
+    # sizes, frames, lengths, classes, kind
+    ([56, 57, 59, 60, 61, 63, 64, 65], 96, [96, 95, 91, 90, 89, 88, 81, 65], 40, "chain"),       # around one strip
+    ([116, 117, 119, 120, 121, 125], 200, [200, 199, 193, 192, 191, 126], 23, "optional"),
+    ([232, 236, 237, 240, 241, 245], 400, [400, 399, 393, 385, 384, 243], 97, "chain"),          # around one workgroup
+    ([480, 476, 481, 477], 700, [700, 697, 480, 699], 300, "optional"),                          # two of them; just enough frames
+    ([1, 2, 3, 4, 5, 8], 24, [24, 1, 7, 8, 9, 17], 5, "chain"),                                  # the smallest
+    ([6, 61, 125, 242, 300], 330, [330, 200, 329, 328, 327], 60, "ctc"),                         # strips with edges of any kind
+    ([70, 130, 250, 64], 180, [180, 179, 177, 64], 31, "wide"),
+    ([70, 130, 250, 64], 280, [280, 279, 277, 64], 31, "far"),                                   # the other kernels
+    ([300, 200, 100], 150, [150, 100, 99], 50, "chain"),                                         # the end is out of reach for two of them
+    ([1900, 1100], 2304, [2301, 1100], 700, "optional"),                                         # many workgroups, several passes of the gather
+]
+
+
+@pytest.mark.parametrize("permute", [False, True], ids=["in_order", "permuted"])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_best_path(oracle, case, permute):
+    sizes, T, lens, F, kind = CASES[case]
+    rng = np.random.default_rng(100 + case)
+    edges, weights, start_end, n = automata(rng, sizes, F, kind, permute)
+    am = -0.25 * rng.integers(0, 12, size=(T, len(sizes), F)).astype(np.float32)      # multiples of 1/4: ties
+    seq_lens = np.array(lens, dtype=np.int32)
+    args = (am, edges, weights, start_end, seq_lens, n)
+    align, scores, _ = run_cabi_viterbi(*args)
+    assert_identical((align, scores), oracle.viterbi_oracle(*args))
+
+
+def test_scores_that_are_not_numbers():
+    """A NaN never wins, -inf closes an edge, a class of +inf takes everything: as in the other kernels (the reference's
+    compare-and-swap does something else with a NaN)."""
+    rng = np.random.default_rng(7)
+    edges, weights, start_end, n = automata(rng, [90, 61, 130], 20, "optional")
+    am = rng.normal(size=(150, 3, 20)).astype(np.float32)
+    am[rng.random(am.shape) < 0.05] = np.nan
+    am[rng.random(am.shape) < 0.05] = -np.inf
+    am[40, 1, 3] = np.inf
+    args = (am, edges, weights, start_end, np.array([150, 149, 141], dtype=np.int32), n)
+    got = run_cabi_viterbi(*args)
+    cabi.set_overlap(1)
+    want = run_cabi_viterbi(*args)
+    assert_identical(got[:2], want[:2])
+    assert np.isfinite(got[1][0]) and np.isposinf(got[1][1]) and np.isneginf(got[1][2])
+
+
+def test_replayed_graph(oracle):
+    """Counters and tables start afresh on every replay of a captured call."""
+    rng = np.random.default_rng(11)
+    edges, weights, start_end, n = automata(rng, [300, 250], 40, "optional")
+    am = rng.normal(size=(420, 2, 40)).astype(np.float32)
+    seq_lens = np.array([420, 400], dtype=np.int32)
+    dev = torch.device("cuda:0")
+    d = [torch.from_numpy(np.ascontiguousarray(x)).to(dev) for x in (am, edges, weights, start_end, seq_lens)]
+    T, B, F = am.shape
+    E = edges.shape[1]
+    align = torch.empty((T, B), dtype=torch.int32, device=dev)
+    scores = torch.empty((B,), dtype=torch.float32, device=dev)
+    ws = torch.empty(cabi.workspace_size(T, B, F, E, n), dtype=torch.uint8, device=dev)
+
+    def call():
+        cabi.viterbi(d[0].data_ptr(), d[0].stride(0), d[0].stride(1), d[1].data_ptr(), d[1].stride(0), d[2].data_ptr(), d[3].data_ptr(),
+                     d[3].stride(0), d[4].data_ptr(), T, B, F, E, n, align.data_ptr(), align.stride(0), align.stride(1), scores.data_ptr(),
+                     ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for i in range(4):
+        am = rng.normal(size=am.shape).astype(np.float32)
+        d[0].copy_(torch.from_numpy(am))
+        align.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_identical((align.cpu().numpy(), scores.cpu().numpy()), oracle.viterbi_oracle(am, edges, weights, start_end, seq_lens, n))
