@@ -71,6 +71,8 @@ constexpr int COMB_XS = 1024;         // edge scores staged in LDS per pass of t
 constexpr int COMB_BATCH = 4;         // frames the row writer takes together for sequences of up to COMB_BATCH_EDGES edges (rows of up to COMB_BATCH_F floats)
 constexpr int COMB_BATCH_EDGES = 512, COMB_BATCH_F = 1024;
 constexpr int COMB_MID_EDGES = 4096;  // up to here a combine workgroup keeps the edges of its sequence in registers ...
+constexpr int COMB_WIDE_EDGES = 4608;    // ... all of them staged at once where the launch has the LDS for it (CombArgs::xs_cap) ...
+static_assert(COMB_WIDE_EDGES / COMB_THREADS % 2 == 0, "two slots to a register");
 constexpr int COMB_MID_SLOTS = 2048;  // ... and the distinct emissions of the sequence spread over its threads' registers
 #ifndef I6_FLOAT_FRAMES
 #define I6_FLOAT_FRAMES 256           // sequences with more frames keep their state vectors in double (with one or two states per thread double
@@ -113,6 +115,7 @@ constexpr float LN2 = 0.693147180559945309f;
 // the strip behind, walking backward), states a strip advances by, largest number of strips of one sequence
 constexpr int STRIP_HALO = 4, STRIP_USE = 64 - STRIP_HALO, STRIP_MAX = (S_MAX + STRIP_HALO + STRIP_USE - 1) / STRIP_USE;
 constexpr int STRIP_FRAMES = 8;       // frames per block of the strip kernels
+constexpr int STRIP_DEGREE = 6;       // edges entering or leaving a state that they hold in registers
 
 struct SeqMeta {
     int edge_begin;   // edges with a smaller sequence index
@@ -133,6 +136,8 @@ __host__ __device__ inline long long round16(long long x) { return (x + 15) & ~1
 // prefix sum over sequences (and no cross-workgroup dependency) is needed.
 __host__ __device__ inline long long state_off(long long edge_begin, int b) { return round16(2 * edge_begin) + 32LL * b; }
 __host__ __device__ inline long long slot_off(long long edge_begin, int b) { return round16(edge_begin) + 32LL * b; }
+// (borders between workgroups of the strip kernels, four strips of 60 states each)
+__host__ __device__ inline long long strip_border_off(long long edge_begin, int b) { return edge_begin / 240 + 2LL * b; }
 // (floats per frame of the strip kernels' score table, see strip_kernels.inc)
 __host__ __device__ inline long long strip_off(long long edge_begin, int b) { return round16(edge_begin + (edge_begin >> 1) + (edge_begin >> 2)) + 272LL * b; }
 // Entries of a sequence's renumbering table (see local_state) and the home position of a state id in it
@@ -142,7 +147,7 @@ __host__ __device__ inline unsigned renum_home(int id, unsigned cap) {
 }
 
 struct Layout {
-    size_t meta, sync, sortflag, seqbegin, eidx, ellA, ellB, crec, cbegin, demis, tband, renum, cflag, wpfx, offA, offB, alpha, beta, gtab, base_total, sprog, etab, total;
+    size_t meta, sync, sortflag, seqbegin, eidx, ellA, ellB, crec, cbegin, demis, tband, renum, cflag, wpfx, offA, offB, alpha, beta, gtab, base_total, sprog, soffs, shalo, etab, total;
     long long ss_total, gg_total;
     int wpfx_stride;      // ints per sequence in the emission rank table (0: F too large for it)
 };
@@ -178,6 +183,8 @@ Layout make_layout(long long T, long long B, long long E, long long F = 1) {
     l.base_total = o;
     // (the strip kernels' share; a call whose workspace ends before it runs without them)
     l.sprog = o;    o = align256(o + sizeof(int) * 2 * STRIP_MAX * B);
+    l.soffs = o;    o = align256(o + sizeof(double) * 2 * STRIP_MAX * B * ((T + 7) / 8));
+    l.shalo = o;    o = align256(o + sizeof(double) * 2 * STRIP_HALO * (strip_border_off(E, (int)B) + 2) * (((size_t)T + 7) & ~(size_t)7));
     l.etab = o;     o = align256(o + sizeof(float) * (strip_off(E, (int)B) + 16) * (((size_t)T + 7) & ~(size_t)7));
     l.total = o;
     return l;
@@ -221,19 +228,75 @@ __device__ inline int rec_class(const SeqMeta& m, const int threads = REC_THREAD
     return 3;
 }
 
+// (beside the largest number of strips, in bits 8 and up of the same argument)
+constexpr int STRIPS_CHAINS = 1, STRIPS_LARGE = 2;
 // Number of strips of a sequence that the strip kernels take (strip_kernels.inc), 0 for all others.  They need states
 // numbered so that no edge leads downward and none raises the number by more than the halo, edges that fit the registers,
 // and tables that fit the sequence's share of the workspace; `most` is what the host has launched waves for.
 __device__ inline int strip_count(const SeqMeta& m, const int b, const int T, const int most) {
     const int d = m.pad >> 8;
-    if (d < 1 || d > STRIP_HALO || seq_error(m) != 0 || m.L == 0 || m.n_edges == 0 || m.Kin > KMAX || m.Kout > KMAX) return 0;
-    const int n = (m.S + STRIP_HALO + STRIP_USE - 1) / STRIP_USE;
-    if (n > most) return 0;
+    if (d < 1 || d > STRIP_HALO || seq_error(m) != 0 || m.L == 0 || m.n_edges == 0 || m.Kin > STRIP_DEGREE || m.Kout > STRIP_DEGREE) return 0;
+    const int n = (m.S + STRIP_HALO + STRIP_USE - 1) / STRIP_USE, mode = most >> 8;
+    if (n > (most & 255)) return 0;
+    // full sum: only where they pay (all from the sequence itself, so that other state ids give the same bits)
+    if (mode == STRIPS_CHAINS && 100 * m.n_edges > 205 * m.S) return 0;
+    if (mode == STRIPS_LARGE && 100 * m.n_edges > 205 * m.S && (m.S <= BIG_STATES || 10 * m.n_edges > 23 * m.S)) return 0;
     if (64LL * (d == 1 ? 2 : 3) * n > strip_off(m.edge_begin + m.n_edges, b + 1) - strip_off(m.edge_begin, b)) return 0;
+    if ((n - 1) / 4 > strip_border_off(m.edge_begin + m.n_edges, b + 1) - strip_border_off(m.edge_begin, b)) return 0;
     // (alpha's area also holds back-pointers and halo values of the best-path search: 80 bytes per strip and frame)
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
     if (80LL * n * T8 > 4LL * T * (state_off(m.edge_begin + m.n_edges, b + 1) - state_off(m.edge_begin, b))) return 0;
     return n;
+}
+
+struct StripRange { int t0, t1; };    // frames a strip walks; t0 is a multiple of STRIP_FRAMES
+
+// Forward: strip j holds the states from 60 j on; a state can matter once it can be reached and while the end state can
+// be reached from it.
+__device__ __forceinline__ StripRange strip_range(const SeqMeta& m, const int j) {
+    const int d = m.pad >> 8, s = m.start_local, e = m.end_local;
+    const int lo = j * STRIP_USE, hi = min(lo + STRIP_USE, m.S) - 1;
+    StripRange r = {0, 0};
+    if (hi < s || lo > e) return r;
+    const int first = lo <= s ? 0 : (lo - s + d - 1) / d - 1;           // the step that may first reach state lo
+    const int last = m.L - (e - min(hi, e) + d - 1) / d;                // v_t of state hi is of use up to t = last
+    r.t0 = first & ~(STRIP_FRAMES - 1);
+    r.t1 = min(m.L, last + 1);
+    if (r.t1 <= r.t0) r.t0 = r.t1 = 0;
+    return r;
+}
+
+// The same for the full sum, in whole blocks of virtual time (see fbw_strips): dir 0 alpha; dir 1 beta, where strip j holds
+// the states from STRIP_USE j - STRIP_HALO on.
+__device__ __forceinline__ StripRange fbw_span(const SeqMeta& m, const int dir, const int j) {
+    if (dir == 0) {
+        StripRange r = strip_range(m, j);
+        r.t1 = (r.t1 + STRIP_FRAMES - 1) & ~(STRIP_FRAMES - 1);
+        return r;
+    }
+    const int d = m.pad >> 8, s = m.start_local, e = m.end_local, NB = (m.L + STRIP_FRAMES - 1) / STRIP_FRAMES;
+    const int lo = max(j * STRIP_USE - STRIP_HALO, 0), hi = min(j * STRIP_USE - STRIP_HALO + STRIP_USE, m.S) - 1;
+    StripRange r = {0, 0};
+    if (hi < s || lo > e) return r;
+    const int tmax = m.L - 1 - (e - min(hi, e) + d - 1) / d, tmin = max(0, (max(lo, s) - s + d - 1) / d - 1);      // rows in which one of them can matter
+    if (tmax < tmin) return r;
+    r.t0 = (NB - 1 - min(tmax + 1, m.L - 1) / STRIP_FRAMES) * STRIP_FRAMES;        // from the step that makes the last of these rows
+    r.t1 = (NB - tmin / STRIP_FRAMES) * STRIP_FRAMES;
+    return r;
+}
+// does strip j walk block q of the sequence?
+__device__ __forceinline__ bool strip_walks(const SeqMeta& m, const int dir, const int j, const int q) {
+    const StripRange r = fbw_span(m, dir, j);
+    const int v = (dir ? (m.L + STRIP_FRAMES - 1) / STRIP_FRAMES - 1 - q : q) * STRIP_FRAMES;
+    return v >= r.t0 && v < r.t1;
+}
+
+// Waves per sequence that a call launches: half as many strips again as the average automaton has and two more (a longer one is
+// the other kernels'), and all a sequence can have while the batch is small (a workgroup without a strip ends at once).
+inline int strips_to_launch(const int B, const int E, const int n_states) {
+    const long long states = std::min((long long)n_states, (long long)E + B) / B + 1;
+    const long long n = std::max((states * 3 / 2 + STRIP_USE - 1) / STRIP_USE + 2, 1024LL / B);
+    return (int)std::min(n, (long long)STRIP_MAX);
 }
 
 // Hand-off between kernels that run at the same time (gather -> recursion -> combine).  The
@@ -332,6 +395,7 @@ struct PrepArgs {
     int* wpfx = nullptr;    // per sequence: number of distinct emissions below 32 * w, for w = 0 .. ceil(F / 32); may be null
     int wpfx_stride = 0;
     int strips = 0;         // > 0: sequences of up to that many strips go to the strip kernels
+    int level = 0;          // 1: every sequence whose ids do not follow the automaton gets numbers along it; 2: those of at most 2.3 edges per state
     int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence
 };
 
@@ -668,7 +732,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
     static_assert(2 * PREP_AUX_WORDS >= S_MAX && S_MAX <= 4096 && EB_MAX >= 2 * S_MAX, "height << 16 | state; sort key height << 12 | state");
     unsigned* dn = ranked ? uniq + LEVEL_STATES : uniq;     // [S]: hops to the end of the chain of chosen successors << 16 | that end
     unsigned short* num = (unsigned short*)aux;              // [S]: the state's number
-    bool by_level = unordered && (ranked || !sparse) && !generic && S <= (ranked ? LEVEL_STATES : S_MAX) && L > 0 && (a.strips > 0 || 5LL * S > 4LL * L);
+    bool by_level = unordered && (ranked || !sparse) && !generic && S <= (ranked ? LEVEL_STATES : S_MAX) && L > 0 && (a.level == 1 || (a.level == 2 && 10LL * n_edges <= 23LL * S) || 5LL * S > 4LL * L);
     if (by_level) {
         unsigned* cand = keys;                    // [S]: (height of the best successor + 1) << 16 | that successor
         constexpr int SPT = S_MAX / NT;           // states per thread
@@ -1117,6 +1181,7 @@ struct RecArgs {
     const SeqMeta* meta; const uint2* ellA; const uint2* ellB; const float* gtab; float* gtab_rw;
     float* alpha; float* beta; double* offA; double* offB;
     int* sync;
+    int strips = 0;       // > 0: sequences of up to that many strips are fbw_strips'
 };
 
 // Barrier for LDS traffic only: waits for this wave's LDS operations and not for its global
@@ -1755,6 +1820,7 @@ __device__ __forceinline__ void recurse_workgroup(const RecArgs& a, float* lds) 
     }
     const int b = blockIdx.x >> 1, dir = blockIdx.x & 1;
     const SeqMeta m = a.meta[b];
+    if (!SYNC && a.strips > 0 && strip_count(m, b, a.T, a.strips) > 0) return;
     const int cls = rec_class(m, T_);
     if (cls == -2) {
         const long long soff = state_off(m.edge_begin, b);
@@ -1855,6 +1921,8 @@ __global__ __launch_bounds__(REC_BLOCK_BIG) void fbw_recurse_big(RecArgs a) {
     recurse_workgroup<SYNC, 2>(a, lds);
 }
 
+#include "strip_kernels.inc"
+
 // ---------------------------------------------------------------------------------------------
 // stage 4: combine.  One workgroup per (strip of TC frames, sequence).  The F-wide row image
 // lives in LDS: its non-hole positions are the same for every frame of a sequence, so it is
@@ -1872,6 +1940,9 @@ struct CombArgs {
     int direct_only;             // beside fbw_flat: only the sequences that kernel leaves to this one (flat_direct)
     int small_elsewhere = 0;     // the sequences of comb_small() are written by the SMALL instance of this kernel, launched beside this one
     int pad_rows = 0;            // the general instance also writes the rows of frames >= seq_len (no fbw_padfill in this call)
+    int xs_cap = 0;              // general instance: edges its staging area holds beyond COMB_XS (0: no more)
+    int strips = 0;              // > 0: sequences of up to that many strips have rows of fbw_strips, with
+    const double* soffs = nullptr;   // an offset per direction, strip and block of frames (+inf: not walked)
     int batch_frames = 0;        // SMALL instance: the LDS of the launch holds COMB_BATCH row images and staging areas (comb_batch_lds_bytes)
 };
 
@@ -1883,6 +1954,60 @@ typedef float float4a __attribute__((ext_vector_type(4)));
 // posterior jobs, fbw_combine (row by row, started beside it with direct_only set) for the larger
 // ones and for those on the general path.  Sequences with a reported problem or without edges have
 // constant rows, which the write jobs of fbw_flat produce by themselves.
+// The rows of fbw_strips are relative to an offset per strip and block of frames.  For a block, the offsets of the two rows
+// that an edge joins (alpha of the strip that holds its source, beta of the one that holds its target, which is the same
+// strip or the next) become part of the edge's weight, relative to the smallest sum of two such offsets; that sum takes
+// the place of the row offsets.  An edge one of whose strips does not walk the block is dead there: weight +inf, and its
+// operands are taken from rows that were written.
+struct StripView {
+    float dist[2 * STRIP_MAX];     // by strip of the source + strip of the target
+    double base;
+    unsigned safe;                 // source | target << 16 of written rows
+};
+__device__ __forceinline__ bool strip_view(StripView& v, const CombArgs& a, const SeqMeta& m, const int b, const int q) {
+    const int n = a.strips > 0 ? strip_count(m, b, a.T, a.strips) : 0;
+    if (n == 0) return false;
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x, nblkT = (a.T + STRIP_FRAMES - 1) / STRIP_FRAMES;
+        const double* offA = a.soffs + (size_t)(2 * b) * STRIP_MAX * nblkT + q;
+        const double* offB = offA + (size_t)STRIP_MAX * nblkT;
+        double base = INF_F, sum[3];
+        unsigned sa = 0xffffu, sb = 0xffffu;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int k = lane + 64 * i, ja = k >> 1, jb = ja + (k & 1);
+            sum[i] = INF_F;
+            if (64 * i >= 2 * n) break;
+            if (ja < n && jb < n) {
+                const double oa = offA[(size_t)ja * nblkT], ob = offB[(size_t)jb * nblkT];
+                sum[i] = oa + ob;
+                if (oa < (double)INF_F) sa = min(sa, (unsigned)(ja * STRIP_USE));
+                if (ob < (double)INF_F) sb = min(sb, (unsigned)max(jb * STRIP_USE - STRIP_HALO, 0));
+            }
+            base = __builtin_fmin(base, sum[i]);
+        }
+        for (int x = 1; x < 64; x <<= 1) {
+            base = __builtin_fmin(base, __shfl_xor(base, x));
+            sa = min(sa, (unsigned)__shfl_xor((int)sa, x));
+            sb = min(sb, (unsigned)__shfl_xor((int)sb, x));
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (lane + 64 * i < 2 * n) v.dist[lane + 64 * i] = sum[i] < (double)INF_F ? (float)(sum[i] - base) : INF_F;
+        if (lane == 0) {
+            v.base = base < (double)INF_F ? base : 0.0;
+            v.safe = (sa == 0xffffu ? 0u : sa) | ((sb == 0xffffu ? 0u : sb) << 16);
+        }
+    }
+    __syncthreads();
+    return true;
+}
+__device__ __forceinline__ void strip_edge(const StripView& v, uint4& r) {
+    const float d = v.dist[(r.x & 0xFFFFu) / STRIP_USE + ((r.x >> 16) + STRIP_HALO) / STRIP_USE];
+    r.y = __float_as_uint(__uint_as_float(r.y) + d);
+    if (d == INF_F) r.x = v.safe;
+}
+
 constexpr int COMB_FAST_EDGES = 1024, COMB_FAST_SLOTS = 512;
 // (fbw_flat: up to COMB_FAST_* everything of a thread stays in registers over the frames of a job; up to
 // FLAT_* the edges are taken in pieces of COMB_FAST_EDGES per frame, their scores parked in the staging area)
@@ -2135,7 +2260,8 @@ __device__ __forceinline__ bool comb_small(const SeqMeta& m, const int batch) {
 #define I6_COMB_SMALL_OCC 6
 #endif
 constexpr int COMB_SMALL_OCC = I6_COMB_SMALL_OCC;
-template <bool SYNC, bool NEGLOG, bool SMALL = false>
+// (WIDE: the general instance with the path for more than COMB_XS staged edges in the place of the one in passes)
+template <bool SYNC, bool NEGLOG, bool SMALL = false, bool WIDE = false>
 __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_combine(CombArgs a) {
     extern __shared__ float4a lds4[];
     __shared__ float redmin[COMB_THREADS / 64];
@@ -2237,6 +2363,8 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
     const float* abase = a.alpha + (size_t)T * soff;
     const float* bbase = a.beta + (size_t)T * soff;
     const float* gbase = a.gtab + (size_t)T * goff;
+    __shared__ StripView view;
+    const bool stripped = !SYNC && strip_view(view, a, m, b, t0 / STRIP_FRAMES);
 
     // writes the image positions of one frame from the per-slot sums (sd: sums of probabilities relative to
     // the frame minimum; NEGLOG: ls, the sums in log space), then streams the row out
@@ -2319,6 +2447,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             const int i = tid + j * COMB_THREADS;
             uint4 r = make_uint4(0u, __float_as_uint(INF_F), 0u, 0u);     // weight +inf: contributes nothing
             if (i < nE) r = crec[i];
+            if (stripped) strip_edge(view, r);
             eft[j] = r.x; esl[j] = r.z; ew[j] = __uint_as_float(r.y);
         }
         int c0[JS], c1[JS], em[JS];
@@ -2334,7 +2463,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             // operands of all frames of the batch in one round trip (frames past the end: the last one once more, unused)
             float x[MF][JE], lmin[MF];
             // the row offsets: lane 2f has the alpha row's of frame f, lane 2f+1 the beta row's
-            const double voff = tid < 2 * nf ? load_x<SYNC>(((tid & 1) ? offB : offA) + tb + (tid >> 1)) : 0.0;
+            const double voff = tid >= 2 * nf ? 0.0 : stripped ? ((tid & 1) ? 0.0 : view.base) : load_x<SYNC>(((tid & 1) ? offB : offA) + tb + (tid >> 1));
             {
                 float va[MF][JE], vb[MF][JE], vg[MF][JE];
 #pragma unroll
@@ -2467,6 +2596,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             const int i = tid + j * COMB_THREADS;
             uint4 r = make_uint4(0u, __float_as_uint(INF_F), 0u, 0u);     // weight +inf: contributes nothing
             if (i < nE) r = crec[i];
+            if (stripped) strip_edge(view, r);
             efr[j] = r.x & 0xFFFFu; eto[j] = r.x >> 16; esl[j] = r.z; ew[j] = __uint_as_float(r.y);
         }
         int c0[JS], c1[JS], em[JS];
@@ -2486,7 +2616,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             for (int j = 0; j < JE; j++) {
                 va[j] = load_x<SYNC>(arow + efr[j]); vb[j] = load_x<SYNC>(brow + eto[j]); vg[j] = load_x<SYNC>(grow + esl[j]);
             }
-            if (tid == 0) voff = load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t);
+            if (tid == 0) voff = stripped ? view.base : load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t);
         };
         fetch(t0);
         for (int t = t0; t < tv; t++) {
@@ -2523,7 +2653,64 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             if (!NEGLOG) tot = block_sum256(part, redsum);
             finish_row(t, mn, tot, sd, ls, em, JS, offs);
         }
-    } else if (!SMALL && nE <= COMB_MID_EDGES && D <= COMB_MID_SLOTS) {
+    } else if (WIDE && nE <= a.xs_cap && D <= COMB_MID_SLOTS) {
+        // the same with a staging area for all edges of the sequence (the host sizes it where the average automaton has more
+        // than COMB_XS; posterior modes only, sums in log space would spill): one pass, three barriers a frame, and the registers of a slot's range are read once
+        constexpr int JE = COMB_WIDE_EDGES / COMB_THREADS, JS = COMB_MID_SLOTS / COMB_THREADS;
+        unsigned eft[JE], esl[JE / 2];         // (two slots to a register)
+        float ew[JE];
+#pragma unroll
+        for (int j = 0; j < JE; j++) {
+            const int i = tid + j * COMB_THREADS;
+            uint4 r = make_uint4(0u, __float_as_uint(INF_F), 0u, 0u);     // weight +inf: contributes nothing
+            if (i < nE) r = crec[i];
+            if (stripped) strip_edge(view, r);
+            eft[j] = r.x; ew[j] = __uint_as_float(r.y);
+            esl[j / 2] = (j & 1) ? esl[j / 2] | (r.z << 16) : r.z;
+            if (j % 6 == 5) asm volatile("" ::: "memory");
+        }
+        unsigned* crl = (unsigned*)(xs + COMB_WIDE_EDGES);      // first edge | one past the last edge << 16 of my slots (in LDS, registers are short)
+        int em[JS];
+#pragma unroll
+        for (int js = 0; js < JS; js++) {
+            const int d = tid + js * COMB_THREADS;
+            em[js] = d < D ? de[d] : 0;
+            crl[d] = d < D ? (unsigned)cb[d] | ((unsigned)cb[d + 1] << 16) : 0u;
+        }
+        for (int t = t0; t < tv; t++) {
+            const float* arow = abase + (size_t)t * SP;
+            const float* brow = bbase + (size_t)t * SP;
+            const float* grow = gbase + (size_t)t * DP;
+            float lmin = INF_F;
+#pragma unroll
+            for (int j = 0; j < JE; j++) {
+                const float x = (load_x<SYNC>(arow + (eft[j] & 0xFFFFu)) + ew[j]) + (load_x<SYNC>(grow + ((esl[j / 2] >> (16 * (j & 1))) & 0xFFFFu)) + load_x<SYNC>(brow + (eft[j] >> 16)));
+                xs[tid + j * COMB_THREADS] = x;          // (each thread its own, until the barrier behind the loop below)
+                lmin = fminf(lmin, x);
+                if (j % 3 == 2) asm volatile("" ::: "memory");       // (the operands of three edges in flight: those of all do not fit the registers)
+            }
+            const double offs = tid != 0 ? 0.0 : stripped ? view.base : load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t);
+            const float mn = block_min256(lmin, redmin);
+            float part = 0.f;         // see the fast path
+#pragma unroll
+            for (int j = 0; j < JE; j++) {
+                const float pr = mn == INF_F ? 0.f : __builtin_amdgcn_exp2f(mn - xs[tid + j * COMB_THREADS]);
+                xs[tid + j * COMB_THREADS] = pr;
+            }
+            __syncthreads();
+            float sd[JS];
+#pragma unroll
+            for (int js = 0; js < JS; js++) {
+                const unsigned cr = crl[tid + js * COMB_THREADS];
+                const int e0 = (int)(cr & 0xFFFFu), e1 = (int)(cr >> 16);
+                sd[js] = slot_sum(xs, e0, e1);
+                part += sd[js];
+                if (js & 1) asm volatile("" ::: "memory");
+            }
+            const float tot = block_sum256(part, redsum);
+            finish_row(t, mn, tot, sd, nullptr, em, JS, offs);
+        }
+    } else if (!SMALL && !WIDE && nE <= COMB_MID_EDGES && D <= COMB_MID_SLOTS) {
         // medium sequences: this thread's edges still stay in registers for the whole strip (sixteen
         // of them, source and target packed), the operands of a frame are fetched in one go, and the
         // scores go through the LDS staging area in up to four passes
@@ -2535,6 +2722,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             const int i = tid + j * COMB_THREADS;
             uint4 r = make_uint4(0u, __float_as_uint(INF_F), 0u, 0u);     // weight +inf: contributes nothing
             if (i < nE) r = crec[i];
+            if (stripped) strip_edge(view, r);
             eft[j] = r.x; esl[j] = r.z; ew[j] = __uint_as_float(r.y);
         }
         int em[JS];
@@ -2555,7 +2743,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
                 x[j] = (load_x<SYNC>(arow + (eft[j] & 0xFFFFu)) + ew[j]) + (load_x<SYNC>(grow + esl[j]) + load_x<SYNC>(brow + (eft[j] >> 16)));
                 lmin = fminf(lmin, x[j]);
             }
-            const double offs = tid == 0 ? load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t) : 0.0;
+            const double offs = tid != 0 ? 0.0 : stripped ? view.base : load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t);
             const float mn = block_min256(lmin, redmin);
             float sd[JS];
             LogSum ls[JS];
@@ -2599,7 +2787,8 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
             const float* brow = bbase + (size_t)t * SP;
             const float* grow = gbase + (size_t)t * DP;
             auto score = [&](int i) {
-                const uint4 r = crec[i];
+                uint4 r = crec[i];
+                if (stripped) strip_edge(view, r);
                 return (load_x<SYNC>(arow + (r.x & 0xFFFFu)) + __uint_as_float(r.y)) + (load_x<SYNC>(grow + r.z) + load_x<SYNC>(brow + (r.x >> 16)));
             };
             float lmin = INF_F;
@@ -2637,7 +2826,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
                 if (!NEGLOG) part += sd[jd];
             }
             const float tot = block_sum256(part, redsum);
-            finish_row(t, mn, tot, sd, ls, em, COMB_JD, load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t));
+            finish_row(t, mn, tot, sd, ls, em, COMB_JD, stripped ? view.base : load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t));
         }
     }
 }
@@ -2768,6 +2957,8 @@ __device__ __forceinline__ void flat_post(const FlatArgs& fa, const int b, const
     const float* bbase = a.beta + (size_t)T * soff;
     const float* gbase = a.gtab + (size_t)T * goff;
     float* cpbase = fa.cp + (size_t)T * goff;
+    __shared__ StripView view;
+    const bool stripped = !SYNC && strip_view(view, a, m, b, t0 / STRIP_FRAMES);
 
     constexpr int JE = COMB_FAST_EDGES / COMB_THREADS;
     if (nE > COMB_FAST_EDGES || D > COMB_FAST_SLOTS) {
@@ -2789,7 +2980,7 @@ __device__ __forceinline__ void flat_post(const FlatArgs& fa, const int b, const
 #pragma unroll
         for (int f = 0; f < FLAT_TCF; f++) {
             lmins[f] = INF_F; voffs[f] = 0.0;
-            if (tid == 0 && f < nf) voffs[f] = load_x<SYNC>(offA + t0 + f) + load_x<SYNC>(offB + t0 + f);
+            if (tid == 0 && f < nf) voffs[f] = stripped ? view.base : load_x<SYNC>(offA + t0 + f) + load_x<SYNC>(offB + t0 + f);
         }
         for (int c0 = 0; c0 < nE; c0 += COMB_FAST_EDGES) {
             uint4 r[JE];
@@ -2799,6 +2990,7 @@ __device__ __forceinline__ void flat_post(const FlatArgs& fa, const int b, const
                 const int i = c0 + tid + j * COMB_THREADS;
                 r[j] = make_uint4(0u, __float_as_uint(INF_F), 0u, 0u);     // weight +inf: contributes nothing
                 if (i < nE) r[j] = crec[i];
+                if (stripped) strip_edge(view, r[j]);
             }
 #pragma unroll
             for (int f = 0; f < FLAT_TCF; f++) {
@@ -2882,6 +3074,7 @@ __device__ __forceinline__ void flat_post(const FlatArgs& fa, const int b, const
         const int i = tid + j * COMB_THREADS;
         uint4 r = make_uint4(0u, __float_as_uint(INF_F), 0u, 0u);     // weight +inf: contributes nothing
         if (i < nE) r = crec[i];
+        if (stripped) strip_edge(view, r);
         eft[j] = r.x; esl[j] = r.z; ew[j] = __uint_as_float(r.y);
     }
     unsigned cr[JS];          // first edge | one past the last edge << 16 of my slots
@@ -2901,7 +3094,7 @@ __device__ __forceinline__ void flat_post(const FlatArgs& fa, const int b, const
         for (int j = 0; j < JE; j++) {
             va[j] = load_x<SYNC>(arow + (eft[j] & 0xFFFFu)); vb[j] = load_x<SYNC>(brow + (eft[j] >> 16)); vg[j] = load_x<SYNC>(grow + esl[j]);
         }
-        if (tid == 0) voff = load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t);
+        if (tid == 0) voff = stripped ? view.base : load_x<SYNC>(offA + t) + load_x<SYNC>(offB + t);
     };
     fetch(t0);
     for (int t = t0; t < tv; t++) {
@@ -3339,6 +3532,7 @@ void launch_combine(const bool neglog, const dim3 grid, const size_t lds, hipStr
         ca.small_elsewhere = 1;
     }
     if (neglog) hipLaunchKernelGGL((fbw_combine<SYNC, true, false>), grid, dim3(COMB_THREADS), lds, s, ca);
+    else if (!SYNC && ca.xs_cap) hipLaunchKernelGGL((fbw_combine<false, false, false, true>), grid, dim3(COMB_THREADS), lds, s, ca);
     else hipLaunchKernelGGL((fbw_combine<SYNC, false, false>), grid, dim3(COMB_THREADS), lds, s, ca);
 }
 template <bool SYNC>
@@ -3360,8 +3554,8 @@ int device_init(Pipeline& p) {
     for (const void* k : {(const void*)fbw_combine<true, false, false>, (const void*)fbw_combine<false, false, false>,
                           (const void*)fbw_combine<true, true, false>, (const void*)fbw_combine<false, true, false>,
                           (const void*)fbw_combine<true, false, true>, (const void*)fbw_combine<false, false, true>,
-                          (const void*)fbw_combine<true, true, true>, (const void*)fbw_combine<false, true, true>})
-        HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256));
+                          (const void*)fbw_combine<true, true, true>, (const void*)fbw_combine<false, true, true>, (const void*)fbw_combine<false, false, false, true>})
+        HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048));
     hipFuncAttributes attr;
     HIP_TRY(hipFuncGetAttributes(&attr, (const void*)fbw_recurse_dense<true>));
     p.dense_regs = attr.numRegs;
@@ -3583,8 +3777,11 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // rows too long for the LDS image of the dense write go through it in tiles; so do rows of more
     // than two tiles that would still fit (the smaller image leaves room for three workgroups on a
     // compute unit instead of one or two: 1-2 % faster)
-    const bool tiled = comb_lds_bytes(F) > 160 * 1024 - 256 || F > 2 * COMB_TILE_W;
-    const size_t comb_lds = tiled ? (size_t)COMB_TILE_W * 4 + (size_t)COMB_XS * 4 : comb_lds_bytes(F);
+    const bool tiled = comb_lds_bytes(F) > 160 * 1024 - 2048 || F > 2 * COMB_TILE_W;
+    // automata of more than COMB_XS edges on average: the general instance of the row writer stages all edges of a frame
+    // (but for rows so long that the image leaves room for a single workgroup)
+    bool wide = out_mode != I6FBW_OUT_NEG_LOG && (long long)E > (long long)COMB_XS * B && (tiled || F <= COMB_TILE_W);
+    size_t comb_lds = tiled ? (size_t)COMB_TILE_W * 4 + (size_t)COMB_XS * 4 : comb_lds_bytes(F);
 
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
@@ -3616,6 +3813,18 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // 0.34, T=4000 B=8 with large automata: 3.27 / 2.81).
     bool overlap = forced >= 0 ? forced != 0
                                : ((long long)T * B * F >= (1LL << 26) && 2 * B <= P.n_cu / 2 && T >= 384 && (B >= 12 || T >= 1000));
+    // The strip kernels take the place of the recursion stage after stage: also where the overlap would pay for the large
+    // instance.  (The dump of the forward scores reads rows in the layout of the other kernels.)
+    // They pay for chains (two candidates per state: 115 ns a frame where fbw_recurse takes 170) and for large automata with
+    // optional states (180 instead of 680), not for small ones with three candidates (172 / 196 ns, but a larger gather) nor
+    // for CTC, whose last strip has edges of any kind (540 ns).  The device decides sequence by sequence (strip_count); here
+    // only whether any of them can be meant.
+    const bool strips_large = (long long)E > 1100LL * B;
+    const bool strips_pay = T >= 256 && (100LL * E <= 205LL * n_states || (strips_large && 10LL * E <= 23LL * n_states));
+    int strips = strips_pay && !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strips_to_launch(B, E, n_states) : 0;
+    const int strip_waves = strips;
+    if (strips > 0) strips |= (strips_large ? STRIPS_LARGE : STRIPS_CHAINS) << 8;
+    if (strips > 0 && strips_large && big && forced < 0) overlap = false;
     // All 2B recursion workgroups must be on the machine at the same time (at most two per compute
     // unit): gather and dense write wait for their progress while occupying wave slots themselves.
     if (2 * B > (dense ? 2 : 1) * P.n_cu) overlap = false;
@@ -3627,6 +3836,8 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // leave no room for the gather's waves, which they wait for.  (The compiler is asked for 96; how
     // close it gets depends on its version.)
     if (dense && P.dense_regs > 104) overlap = false;
+    // (a call that overlaps by its sizes keeps the same recursion, and the same bits, where capture or busy streams keep it from it)
+    if (overlap) strips = 0;
     if (overlap) {
         // under stream capture: one stream, no in-memory waits between kernels, no synchronisation
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -3649,6 +3860,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     pa.ellA = (uint2*)(ws + l.ellA); pa.ellB = (uint2*)(ws + l.ellB);
     pa.crec = (uint4*)(ws + l.crec); pa.cbegin = (int*)(ws + l.cbegin); pa.demis = (int*)(ws + l.demis); pa.tband = (int2*)(ws + l.tband);
     pa.cflag = (int*)(ws + l.cflag); pa.wpfx = l.wpfx_stride > 0 ? (int*)(ws + l.wpfx) : nullptr; pa.wpfx_stride = l.wpfx_stride;
+    pa.strips = strips; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog);
     GatherArgs ga;
     ga.am = am; ga.st_t = am_stride_t; ga.st_b = am_stride_b; ga.T = T; ga.B = B;
     ga.meta = meta; ga.demis = pa.demis; ga.tband = pa.tband; ga.gtab = (float*)(ws + l.gtab); ga.sync = sync;
@@ -3661,6 +3873,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     ra.gen = gen;
     ra.T = T; ra.B = B; ra.prep_wgs = 3 * B; ra.meta = meta; ra.ellA = pa.ellA; ra.ellB = pa.ellB; ra.gtab = ga.gtab; ra.gtab_rw = ga.gtab;
     ra.alpha = (float*)(ws + l.alpha); ra.beta = (float*)(ws + l.beta);
+    ra.strips = strips;
     ra.offA = (double*)(ws + l.offA); ra.offB = (double*)(ws + l.offB); ra.sync = sync;
     CombArgs ca;
     ca.gen = gen;
@@ -3670,6 +3883,10 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     ca.out = out; ca.sum_output = sum_output; ca.ost_t = out_stride_t; ca.ost_b = out_stride_b; ca.sync = sync;
     ca.tile_w = tiled ? COMB_TILE_W : 0;
     ca.direct_only = 0;
+    wide = wide && !overlap;
+    if (wide) comb_lds += (size_t)(COMB_WIDE_EDGES - COMB_XS + COMB_MID_SLOTS) * 4;
+    ca.xs_cap = wide ? COMB_WIDE_EDGES : 0;
+    ca.strips = strips; ca.soffs = (const double*)(ws + l.soffs);
     // The dense tensor goes out in flat spans (fbw_flat) if it is one contiguous block in either
     // order of frames and sequences, rows are long enough for a span to cut at most two of them,
     // and the tensor is large (for small problems the row writer is as good).
@@ -3775,7 +3992,20 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     if (overlap) HIP_TRY(hipEventRecord(P.doneP, sP));
 
     if (!overlap) {
-        { StageTimer tm(1, s, timed); hipLaunchKernelGGL(fbw_gather<false>, g_grid, dim3(256), 0, s, ga); }
+        if (strips > 0) {
+            StripGatherArgs sg;
+            sg.g = ga; sg.ell = pa.ellA; sg.etab = (float*)(ws + l.etab); sg.strips = strips; sg.cap = strip_gather_lds(B, E); sg.keep_rows = 1; sg.soffs = (double*)(ws + l.soffs);
+            FbwStripArgs sa;
+            sa.T = T; sa.B = B; sa.strips = strips; sa.meta = meta; sa.ellA = pa.ellA; sa.ellB = pa.ellB; sa.gtab = ga.gtab; sa.etab = sg.etab;
+            sa.alpha = ra.alpha; sa.beta = ra.beta; sa.soffs = sg.soffs; sa.halo = (double*)(ws + l.shalo); sa.prog = pa.sprog; sa.sync = sync;
+            { StageTimer tm(1, s, timed); hipLaunchKernelGGL(strip_gather, g_grid, dim3(256), sg.cap * sizeof(float), s, sg); }
+            HIP_TRY(hipGetLastError());
+            StageTimer tm(2, s, timed);
+            hipLaunchKernelGGL(fbw_strips, dim3((unsigned)(2 * B * ((strip_waves + STRIP_WAVES - 1) / STRIP_WAVES))), dim3(STRIP_BLOCK), 0, s, sa);
+        } else {
+            StageTimer tm(1, s, timed);
+            hipLaunchKernelGGL(fbw_gather<false>, g_grid, dim3(256), 0, s, ga);
+        }
         HIP_TRY(hipGetLastError());
         { StageTimer tm(2, s, timed); if (dense) hipLaunchKernelGGL(fbw_recurse_dense<false>, dim3(2 * B), dim3(REC_BLOCK_DENSE), sizeof(float) * REC_LDS_FLOATS_F32, s, ra);
           else if (big) hipLaunchKernelGGL(fbw_recurse_big<false>, dim3(2 * B), dim3(REC_BLOCK_BIG), 0, s, ra);
@@ -4095,6 +4325,5 @@ int i6fbw_profile_read(float* stage_ms) {
 
 }  // extern "C"
 
-#include "strip_kernels.inc"
 #include "viterbi_kernels.inc"
 #include "fsa_builders.inc"

@@ -137,3 +137,28 @@ def test_replayed_graph(oracle):
         graph.replay()
         torch.cuda.synchronize()
         assert_identical((align.cpu().numpy(), scores.cpu().numpy()), oracle.viterbi_oracle(am, edges, weights, start_end, seq_lens, n))
+
+
+FULL_SUM = [
+    ([119, 120, 121, 176, 180, 181], 264, [264, 263, 257, 256, 199, 264], 40, "chain"),      # borders of strips, of blocks, of the last block
+    ([236, 240, 244, 480], 600, [600, 599, 593, 592], 97, "chain"),                          # borders of workgroups
+    ([300, 290, 20], 304, [301, 290, 5], 50, "chain"),                                       # just enough frames; an end out of reach
+    ([700, 650, 1200], 1288, [1288, 1281, 1250], 300, "optional"),                           # large, three sources per state
+]
+
+
+@pytest.mark.parametrize("permute", [False, True], ids=["in_order", "permuted"])
+@pytest.mark.parametrize("case", range(len(FULL_SUM)))
+def test_full_sum(oracle, case, permute):
+    """Losses to 1e-5 and posteriors to 1e-4 of the oracle's, the bars of the other full-sum tests."""
+    from tests.gpu_util import run_cabi
+    from tests.helpers import posterior
+    sizes, T, lens, F, kind = FULL_SUM[case]
+    rng = np.random.default_rng(300 + case)
+    edges, weights, start_end, n = automata(rng, sizes, F, kind, permute)
+    am = rng.uniform(0.1, 9.0, size=(T, len(sizes), F)).astype(np.float32)
+    args = (am, edges, -weights, start_end, np.array(lens, dtype=np.int32), n)
+    want_out, want_loss = oracle.fbw_oracle(*args, threads=4)
+    out, loss = run_cabi(*args)
+    np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(posterior(out), posterior(want_out), rtol=0, atol=1e-4)
