@@ -162,3 +162,23 @@ def test_full_sum(oracle, case, permute):
     out, loss = run_cabi(*args)
     np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
     np.testing.assert_allclose(posterior(out), posterior(want_out), rtol=0, atol=1e-4)
+
+
+def test_last_block_of_a_tight_sequence(oracle):
+    """The last strip holds nothing but the end state, which no row of the last block needs; the frames of that block behind
+    the sequence's end are in nobody's score table (more than 1024 classes: four frames a pass), so they hold what
+    the workspace held.  Neither may show in the results."""
+    from tests.gpu_util import DeviceProblem
+    from tests.helpers import posterior
+    sizes, T, F = [1141, 701], 1140, 12000
+    rng = np.random.default_rng(12)
+    edges, weights, start_end, n = automata(rng, sizes, F, "chain")
+    am = rng.uniform(0.1, 9.0, size=(T, 2, F)).astype(np.float32)
+    args = (am, edges, -weights, start_end, np.array([1140, 700], dtype=np.int32), n)
+    want_out, want_loss = oracle.fbw_oracle(*args, threads=4)
+    P = DeviceProblem(*args)
+    for fill in (-1e30, 1e30):
+        P.ws.view(torch.float32).fill_(fill)
+        out, loss = P.run(cabi.OUT_PROB)
+        np.testing.assert_allclose(loss.cpu().numpy(), want_loss, rtol=1e-5, atol=1e-6)
+        np.testing.assert_allclose(out.cpu().numpy(), posterior(want_out), rtol=0, atol=1e-4)
