@@ -249,6 +249,10 @@ __device__ inline int strip_count(const SeqMeta& m, const int b, const int T, co
     return n;
 }
 
+// Progress counters of a sequence's strips: one per border in either direction, fewer than the 2 * STRIP_MAX there is room
+// for; the last is set when a wait of its strips has run out, which leaves the sequence without values.
+__device__ __forceinline__ bool strip_lost(const int* sprog, const int b) { return sprog[(size_t)(b + 1) * 2 * STRIP_MAX - 1] != 0; }
+
 struct StripRange { int t0, t1; };    // frames a strip walks; t0 is a multiple of STRIP_FRAMES
 
 // Forward: strip j holds the states from 60 j on; a state can matter once it can be reached and while the end state can
@@ -396,7 +400,7 @@ struct PrepArgs {
     int wpfx_stride = 0;
     int strips = 0;         // > 0: sequences of up to that many strips go to the strip kernels
     int level = 0;          // 1: every sequence whose ids do not follow the automaton gets numbers along it; 2: those of at most 2.3 edges per state
-    int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence
+    int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence; the last one is the mark of strip_lost
 };
 
 // sortflag[blk] = 1 if the sequence indices of edges [blk*SCAN_BLOCK, (blk+1)*SCAN_BLOCK] never
@@ -1942,7 +1946,8 @@ struct CombArgs {
     int pad_rows = 0;            // the general instance also writes the rows of frames >= seq_len (no fbw_padfill in this call)
     int xs_cap = 0;              // general instance: edges its staging area holds beyond COMB_XS (0: no more)
     int strips = 0;              // > 0: sequences of up to that many strips have rows of fbw_strips, with
-    const double* soffs = nullptr;   // an offset per direction, strip and block of frames (+inf: not walked)
+    const double* soffs = nullptr;   // an offset per direction, strip and block of frames (+inf: not walked), and
+    const int* sprog = nullptr;      // a mark where they could not be computed (strip_lost)
     int batch_frames = 0;        // SMALL instance: the LDS of the launch holds COMB_BATCH row images and staging areas (comb_batch_lds_bytes)
 };
 
@@ -1963,12 +1968,14 @@ struct StripView {
     float dist[2 * STRIP_MAX];     // by strip of the source + strip of the target
     double base;
     unsigned safe;                 // source | target << 16 of written rows
+    bool lost;                     // the rows could not be computed
 };
 __device__ __forceinline__ bool strip_view(StripView& v, const CombArgs& a, const SeqMeta& m, const int b, const int q) {
     const int n = a.strips > 0 ? strip_count(m, b, a.T, a.strips) : 0;
     if (n == 0) return false;
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x, nblkT = (a.T + STRIP_FRAMES - 1) / STRIP_FRAMES;
+        const bool lost = strip_lost(a.sprog, b);
         const double* offA = a.soffs + (size_t)(2 * b) * STRIP_MAX * nblkT + q;
         const double* offB = offA + (size_t)STRIP_MAX * nblkT;
         double base = INF_F, sum[3];
@@ -1995,6 +2002,7 @@ __device__ __forceinline__ bool strip_view(StripView& v, const CombArgs& a, cons
         for (int i = 0; i < 3; i++)
             if (lane + 64 * i < 2 * n) v.dist[lane + 64 * i] = sum[i] < (double)INF_F ? (float)(sum[i] - base) : INF_F;
         if (lane == 0) {
+            v.lost = lost;
             v.base = base < (double)INF_F ? base : 0.0;
             v.safe = (sa == 0xffffu ? 0u : sa) | ((sb == 0xffffu ? 0u : sb) << 16);
         }
@@ -2365,6 +2373,13 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
     const float* gbase = a.gtab + (size_t)T * goff;
     __shared__ StripView view;
     const bool stripped = !SYNC && strip_view(view, a, m, b, t0 / STRIP_FRAMES);
+    if (stripped && view.lost) {
+        for (int t = t0; t < tv; t++) {
+            stream_const_row(a.out + t * a.ost_t + b * a.ost_b, a.F, __builtin_nanf(""));
+            if (tid == 0) a.sum_output[(size_t)t * B + b] = __builtin_nanf("");
+        }
+        return;
+    }
 
     // writes the image positions of one frame from the per-slot sums (sd: sums of probabilities relative to
     // the frame minimum; NEGLOG: ls, the sums in log space), then streams the row out
@@ -2959,6 +2974,11 @@ __device__ __forceinline__ void flat_post(const FlatArgs& fa, const int b, const
     float* cpbase = fa.cp + (size_t)T * goff;
     __shared__ StripView view;
     const bool stripped = !SYNC && strip_view(view, a, m, b, t0 / STRIP_FRAMES);
+    if (stripped && view.lost) {
+        for (int t = t0 + tid; t < tv; t += COMB_THREADS) a.sum_output[(size_t)t * B + b] = __builtin_nanf("");
+        if (tid == 0) store_agent(flag, 2);
+        return;
+    }
 
     constexpr int JE = COMB_FAST_EDGES / COMB_THREADS;
     if (nE > COMB_FAST_EDGES || D > COMB_FAST_SLOTS) {
@@ -3886,7 +3906,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     wide = wide && !overlap;
     if (wide) comb_lds += (size_t)(COMB_WIDE_EDGES - COMB_XS + COMB_MID_SLOTS) * 4;
     ca.xs_cap = wide ? COMB_WIDE_EDGES : 0;
-    ca.strips = strips; ca.soffs = (const double*)(ws + l.soffs);
+    ca.strips = strips; ca.soffs = (const double*)(ws + l.soffs); ca.sprog = (const int*)(ws + l.sprog);
     // The dense tensor goes out in flat spans (fbw_flat) if it is one contiguous block in either
     // order of frames and sequences, rows are long enough for a span to cut at most two of them,
     // and the tensor is large (for small problems the row writer is as good).

@@ -237,9 +237,11 @@ void i6fbw_set_overlap(int mode);
 void i6fbw_set_band(int on);
 
 /*
- * TEST HOOK, not for production code.  Kernels of the overlapped schedule that wait for another kernel
- * of the same call poll at most `polls` times (default 2^20, restored by polls <= 0) before they give up:
- * the call then reports I6FBW_ERR_TIMEOUT and the rows that could not be computed hold NaN.  It exists so
+ * TEST HOOK, not for production code.  Kernels that wait for another kernel of the same call (the
+ * overlapped schedule), or for another part of the same sequence (the strips of its states), poll at most
+ * `polls` times (default 2^20, restored by polls <= 0; eight times as often where the wait is for LDS)
+ * before they give up: the call then reports I6FBW_ERR_TIMEOUT and the rows that could not be computed hold
+ * NaN (best path: score NaN and an all-zero alignment).  It exists so
  * that a test can force that path from the host (polls = 1) while every kernel still runs to its normal
  * end.  Device-wide for the current device: the call waits for the device to go idle, takes the lock that
  * serialises the library's calls on it, and changes the limit for every call enqueued afterwards by any

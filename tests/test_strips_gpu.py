@@ -182,3 +182,55 @@ def test_last_block_of_a_tight_sequence(oracle):
         out, loss = P.run(cabi.OUT_PROB)
         np.testing.assert_allclose(loss.cpu().numpy(), want_loss, rtol=1e-5, atol=1e-6)
         np.testing.assert_allclose(out.cpu().numpy(), posterior(want_out), rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("writer", [0, 1], ids=["rows", "flat"])
+def test_waits_that_run_out_leave_nan_and_a_status(writer):
+    """Strips that give up waiting for the strip in front of them (a poll limit of one from the host; every wave still walks to its
+    end): the call reports it, rows hold NaN or what they should, and the next call is as ever."""
+    from tests.gpu_util import DeviceProblem
+    rng = np.random.default_rng(5)
+    sizes, T, F = [500, 130, 30], 560, 2500
+    edges, weights, start_end, n = automata(rng, sizes, F, "chain")
+    am = rng.uniform(0.1, 9.0, size=(T, 3, F)).astype(np.float32)
+    P = DeviceProblem(am, edges, -weights, start_end, np.array([560, 551, 540], dtype=np.int32), n)
+    good_out, good_loss = [x.cpu().numpy().copy() for x in P.run(cabi.OUT_PROB)]
+    stream = torch.cuda.current_stream().cuda_stream
+    cabi.set_dense_writer(writer)
+    cabi.set_spin_limit(1)
+    try:
+        P.out.fill_(-7.0)
+        P.loss.fill_(-7.0)
+        P.run(cabi.OUT_PROB, check=False)
+        code, _ = cabi.read_status(P.ws.data_ptr(), P.B, stream)
+    finally:
+        cabi.set_spin_limit(0)
+        cabi.set_dense_writer(-1)
+    out, loss = P.out.cpu().numpy(), P.loss.cpu().numpy()
+    assert code == -15
+    assert np.isnan(out[:, 0]).all() and np.isnan(loss[:, 0]).all()
+    for got, good in ((out, good_out), (loss, good_loss)):
+        np.testing.assert_allclose(got[~np.isnan(got)], good[~np.isnan(got)], rtol=1e-6, atol=1e-6)
+    out, loss = P.run(cabi.OUT_PROB)
+    np.testing.assert_array_equal(out.cpu().numpy(), good_out)
+    np.testing.assert_array_equal(loss.cpu().numpy(), good_loss)
+
+
+def test_best_path_waits_that_run_out(oracle):
+    rng = np.random.default_rng(6)
+    edges, weights, start_end, n = automata(rng, [500, 130, 30], 40, "optional")
+    am = rng.normal(size=(560, 3, 40)).astype(np.float32)
+    args = (am, edges, weights, start_end, np.array([560, 551, 540], dtype=np.int32), n)
+    want = oracle.viterbi_oracle(*args)
+    cabi.set_spin_limit(1)
+    try:
+        align, scores, code = run_cabi_viterbi(*args, check=False)
+    finally:
+        cabi.set_spin_limit(0)
+    assert code == -15 and np.isnan(scores[0])
+    for b in range(3):
+        if np.isnan(scores[b]):
+            assert (align[:, b] == 0).all()
+        else:
+            assert_identical((align[:, b], scores[b:b + 1]), (want[0][:, b], want[1][b:b + 1]))
+    assert_identical(run_cabi_viterbi(*args)[:2], want)
