@@ -46,8 +46,9 @@ def test_ctc_builder_matches_host_generator(seed):
 
 
 # B * Lmax on both sides of FSA_SELF_COUNT (8192: the workgroups count earlier labels themselves, or a kernel in front
-# does), more labels than a workgroup has threads (1024), and sequences without labels
-@pytest.mark.parametrize("B,Lmax", [(1, 1), (3, 1100), (8, 1024), (9, 1024), (300, 2), (1500, 12)])
+# does), more labels than a workgroup has threads (1024, in large batches 128), both sides of FSA_SUM_ONCE (2048 sequences: the
+# earlier sequences' sizes summed by every workgroup or once, 8192 in a round), and sequences without labels
+@pytest.mark.parametrize("B,Lmax", [(1, 1), (3, 1100), (8, 1024), (9, 1024), (300, 2), (1500, 12), (2048, 5), (2049, 5), (2100, 130), (8193, 1)])
 def test_ctc_builder_sizes(B, Lmax):
     from i6_native_ops_amd.fsa import ctc_fsa
     rng = np.random.default_rng(B * 7 + Lmax)
