@@ -103,7 +103,8 @@ constexpr int SEQ_GENERIC = 1;        // value of SeqMeta::err / errA / errB tha
 constexpr int SCAN_BLOCK = 1024;      // edges per workgroup of the sortedness scan
 constexpr int SYNC_HDR = 16;          // ints before the progress counters in the hand-off area:
                                       // [0] abort flag, [1] recursion workgroups placed so far, [3] preparation workgroups finished,
-                                      // [4..5] status report {code, sequence}, [6] longest sequence of the batch in frames
+                                      // [4..5] status report {code, sequence}, [6] longest sequence of the batch in frames,
+constexpr int SYNC_UNCOVERED = 7;     // [7] the batch has a sequence that the strip kernels cannot take
 constexpr int PUBLISH = 32;           // recursion steps between progress publications
 constexpr int SPIN_LIMIT = 1 << 20;   // polls before a waiting wave gives up (see g_spin_limit)
 // Scores are kept in units of log 2 inside the workspace (exp2/log2 are single instructions).
@@ -228,25 +229,33 @@ __device__ inline int rec_class(const SeqMeta& m, const int threads = REC_THREAD
     return 3;
 }
 
-// (beside the largest number of strips, in bits 8 and up of the same argument)
-constexpr int STRIPS_CHAINS = 1, STRIPS_LARGE = 2;
-// Number of strips of a sequence that the strip kernels take (strip_kernels.inc), 0 for all others.  They need states
-// numbered so that no edge leads downward and none raises the number by more than the halo, edges that fit the registers,
-// and tables that fit the sequence's share of the workspace; `most` is what the host has launched waves for.
-__device__ inline int strip_count(const SeqMeta& m, const int b, const int T, const int most) {
-    const int d = m.pad >> 8;
-    if (d < 1 || d > STRIP_HALO || seq_error(m) != 0 || m.L == 0 || m.n_edges == 0 || m.Kin > STRIP_DEGREE || m.Kout > STRIP_DEGREE) return 0;
-    const int n = (m.S + STRIP_HALO + STRIP_USE - 1) / STRIP_USE, mode = most >> 8;
-    if (n > (most & 255)) return 0;
-    // full sum: only where they pay (all from the sequence itself, so that other state ids give the same bits)
-    if (mode == STRIPS_CHAINS && 100 * m.n_edges > 205 * m.S) return 0;
-    if (mode == STRIPS_LARGE && 100 * m.n_edges > 205 * m.S && (m.S <= BIG_STATES || 10 * m.n_edges > 23 * m.S)) return 0;
-    if (64LL * (d == 1 ? 2 : 3) * n > strip_off(m.edge_begin + m.n_edges, b + 1) - strip_off(m.edge_begin, b)) return 0;
-    if ((n - 1) / 4 > strip_border_off(m.edge_begin + m.n_edges, b + 1) - strip_border_off(m.edge_begin, b)) return 0;
+// Number of strips of S states
+__host__ __device__ inline int strips_of(const int S) { return (S + STRIP_HALO + STRIP_USE - 1) / STRIP_USE; }
+// Can the strip kernels (strip_kernels.inc) take an automaton?  They need states numbered so that no edge leads downward (d: by
+// how much one raises the number at most, 0 where that is not so) and none raises the number by more than the halo, and
+// tables that fit the sequence's share of the workspace; `most` is what the host has launched waves for.
+__device__ inline bool strip_shape(const int S, const int n_edges, const int edge_begin, const int b, const int T, const int d, const int most) {
+    const int n = strips_of(S);
+    if (d < 1 || d > STRIP_HALO || n > most) return false;
+    if (64LL * (d == 1 ? 2 : 3) * n > strip_off(edge_begin + n_edges, b + 1) - strip_off(edge_begin, b)) return false;
+    if ((n - 1) / 4 > strip_border_off(edge_begin + n_edges, b + 1) - strip_border_off(edge_begin, b)) return false;
     // (alpha's area also holds back-pointers and halo values of the best-path search: 80 bytes per strip and frame)
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
-    if (80LL * n * T8 > 4LL * T * (state_off(m.edge_begin + m.n_edges, b + 1) - state_off(m.edge_begin, b))) return 0;
-    return n;
+    return 80LL * n * T8 <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
+}
+// A batch goes through the strips as a whole or not at all: with some of its sequences left to the other recursion (or search),
+// which then runs behind the strips, a call took as long as both (8 sequences of 510-690 states, some of them on the other
+// path: 494 us, against 394 without strips and 280 with all of them there).  The preparation's workgroups set the word where
+// one of them finds a sequence that the strips cannot take -- its shape, or a state with more edges than fit the registers;
+// sequences that nothing is computed for do not count.
+// (An unconditional load: it is under way together with the sequence's record.)
+__device__ __forceinline__ bool strips_on(const int strips, const int* sync) {
+    const int uncovered = sync[SYNC_UNCOVERED];
+    return (strips > 0) & (uncovered == 0);
+}
+// Number of strips of a sequence where they are on; 0 where nothing is computed for it.
+__device__ __forceinline__ int strip_count(const SeqMeta& m, const bool on) {
+    return !on || seq_error(m) != 0 || m.L == 0 || m.n_edges == 0 ? 0 : strips_of(m.S);
 }
 
 // Progress counters of a sequence's strips: one per border in either direction, fewer than the 2 * STRIP_MAX there is room
@@ -295,13 +304,14 @@ __device__ __forceinline__ bool strip_walks(const SeqMeta& m, const int dir, con
     return v >= r.t0 && v < r.t1;
 }
 
-// Waves per sequence that a call launches: half as many strips again as the average automaton has and two more (a longer one is
-// the other kernels'), and all a sequence can have while the batch is small (a workgroup without a strip ends at once).
-inline int strips_to_launch(const int B, const int E, const int n_states) {
-    const long long states = std::min((long long)n_states, (long long)E + B) / B + 1;
-    const long long n = std::max((states * 3 / 2 + STRIP_USE - 1) / STRIP_USE + 2, 1024LL / B);
+// Waves per sequence that a call launches: half as many strips again as the average automaton has and two more (with a longer one
+// the batch is the other kernels'), and all a sequence can have while the batch is small (a workgroup without a strip ends at once).
+inline int strips_to_launch(const int B, const long long average_states) {
+    const long long n = std::max((average_states * 3 / 2 + STRIP_USE - 1) / STRIP_USE + 2, 1024LL / B);
     return (int)std::min(n, (long long)STRIP_MAX);
 }
+// The average in a full sum over strips, where the automata have about two edges per state, from the edges alone: see strip_density
+inline long long strip_states(const int B, const int E) { return ((long long)E + B) / (2LL * B) + 1; }
 
 // Hand-off between kernels that run at the same time (gather -> recursion -> combine).  The
 // L2 caches of the eight XCDs are not coherent with each other inside a kernel, so everything
@@ -398,8 +408,9 @@ struct PrepArgs {
     int* cflag = nullptr;   // per (sequence, strip of TC frames): compact posteriors written (flat dense write); may be null
     int* wpfx = nullptr;    // per sequence: number of distinct emissions below 32 * w, for w = 0 .. ceil(F / 32); may be null
     int wpfx_stride = 0;
-    int strips = 0;         // > 0: sequences of up to that many strips go to the strip kernels
-    int level = 0;          // 1: every sequence whose ids do not follow the automaton gets numbers along it; 2: those of at most 2.3 edges per state
+    int strips = 0;         // > 0: a batch of sequences of up to that many strips goes to the strip kernels ...
+    int strip_density = 0;  // ... if none has more than this many edges per 100 states (0: any number)
+    int level = 0;          // 1: every sequence whose ids do not follow the automaton gets numbers along it; 2: those of at most strip_density edges per 100 states
     int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence; the last one is the mark of strip_lost
 };
 
@@ -736,7 +747,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
     static_assert(2 * PREP_AUX_WORDS >= S_MAX && S_MAX <= 4096 && EB_MAX >= 2 * S_MAX, "height << 16 | state; sort key height << 12 | state");
     unsigned* dn = ranked ? uniq + LEVEL_STATES : uniq;     // [S]: hops to the end of the chain of chosen successors << 16 | that end
     unsigned short* num = (unsigned short*)aux;              // [S]: the state's number
-    bool by_level = unordered && (ranked || !sparse) && !generic && S <= (ranked ? LEVEL_STATES : S_MAX) && L > 0 && (a.level == 1 || (a.level == 2 && 10LL * n_edges <= 23LL * S) || 5LL * S > 4LL * L);
+    bool by_level = unordered && (ranked || !sparse) && !generic && S <= (ranked ? LEVEL_STATES : S_MAX) && L > 0 && (a.level == 1 || (a.level == 2 && 100LL * n_edges <= (long long)a.strip_density * S) || 5LL * S > 4LL * L);
     if (by_level) {
         unsigned* cand = keys;                    // [S]: (height of the best successor + 1) << 16 | that successor
         constexpr int SPT = S_MAX / NT;           // states per thread
@@ -905,7 +916,9 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         // bits 8 and up: see below
         m->pad = (sorted ? 1 : 0) | ((sparse || ranked || by_level) ? 2 : 0) | (plain_table ? 4 : 0);
     }
+    auto uncovered = [&]() { if (a.strips > 0 && L > 0 && tid == 0) atomicOr(&a.sync[SYNC_UNCOVERED], 1); };
     if (err || generic || n_edges == 0) {
+        if (!err && n_edges > 0) uncovered();
         if (tid == 0) {
             if (role == 0) { a.meta[b].Kin = 0; a.meta[b].errA = 0; }
             if (role == 1) { a.meta[b].Kout = 0; a.meta[b].errB = 0; }
@@ -985,6 +998,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         const long long share = state_off((long long)edge_begin + n_edges, b + 1) - soff;
         const bool fits = K <= KMAX || (K <= KWIDE && (long long)K * SP <= (long long)KMAX * share);
         const int kerr = fits ? 0 : SEQ_GENERIC;
+        if (K > STRIP_DEGREE) uncovered();
         if (tid == 0) {
             if (role == 0) { a.meta[b].Kin = K; a.meta[b].errA = kerr; }
             else { a.meta[b].Kout = K; a.meta[b].errB = kerr; }
@@ -1041,7 +1055,11 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         dmax = s_dmax; dmin = s_dmin;
         const int s_loc = start_loc, e_loc = end_loc;
         // for the recursion's renormalisation (see live_window): no edge lowers the state number, none raises it by more than dmax
-        if (tid == 0 && dmin == 0 && dmax > 0 && dmax < (1 << 20) && s_loc <= e_loc) a.meta[b].pad |= dmax << 8;
+        const int d = dmin == 0 && dmax > 0 && dmax < (1 << 20) && s_loc <= e_loc ? dmax : 0;
+        if (tid == 0 && d > 0) a.meta[b].pad |= d << 8;
+        // (the states counted here: n_states, which the host has, can be any number of times as large where ids are spread, and the
+        // same automaton is to take the same kernels, and give the same bits, whatever its ids)
+        if (!strip_shape((int)S, n_edges, edge_begin, b, a.T, d, a.strips) || (a.strip_density > 0 && 100LL * n_edges > (long long)a.strip_density * S)) uncovered();
         // one thread per edge; the per-slot minimum / maximum is taken with LDS atomics in the
         // memory of the sort keys (and of the distinct ids of a renumbered sequence), which is not
         // needed any more once each thread has worked out the frames of its own edges
@@ -1120,6 +1138,7 @@ struct GatherArgs {
     float scale;      // log2(e) for -log scores, -log2(e) for log scores
     int ascending;    // strips in ascending order (one consumer walking forward) instead of from both ends inwards
     float fill = INF_F;   // value outside the band: one that never contributes
+    int strips = 0;       // overlapped schedule: > 0: nothing to do for a batch that the strip kernels take, behind these kernels
 };
 
 template <bool SYNC>
@@ -1165,7 +1184,9 @@ __global__ __launch_bounds__(256) void fbw_gather(GatherArgs a) {
 #ifdef I6_TRACE
     trace_corun(3110);
 #endif
+    const bool elsewhere = SYNC && strips_on(a.strips, a.sync);
     const SeqMeta m = a.meta[b];
+    if (elsewhere) return;
     gather_rows<SYNC>(a, m, b, y);
 }
 
@@ -1185,7 +1206,7 @@ struct RecArgs {
     const SeqMeta* meta; const uint2* ellA; const uint2* ellB; const float* gtab; float* gtab_rw;
     float* alpha; float* beta; double* offA; double* offB;
     int* sync;
-    int strips = 0;       // > 0: sequences of up to that many strips are fbw_strips'
+    int strips = 0;       // > 0: nothing to do for a batch that fbw_strips takes
 };
 
 // Barrier for LDS traffic only: waits for this wave's LDS operations and not for its global
@@ -1822,9 +1843,10 @@ __device__ __forceinline__ void recurse_workgroup(const RecArgs& a, float* lds) 
         if (!*go_flag) return;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");      // (and the acquire half all the reader needs: no write-back of the L2 by every wave)
     }
+    // (overlapped: only where the automata are large, see run_impl)
+    if ((!SYNC || INST == 2) && a.strips > 0 && load_x<SYNC>(a.sync + SYNC_UNCOVERED) == 0) return;
     const int b = blockIdx.x >> 1, dir = blockIdx.x & 1;
     const SeqMeta m = a.meta[b];
-    if (!SYNC && a.strips > 0 && strip_count(m, b, a.T, a.strips) > 0) return;
     const int cls = rec_class(m, T_);
     if (cls == -2) {
         const long long soff = state_off(m.edge_begin, b);
@@ -1945,11 +1967,18 @@ struct CombArgs {
     int small_elsewhere = 0;     // the sequences of comb_small() are written by the SMALL instance of this kernel, launched beside this one
     int pad_rows = 0;            // the general instance also writes the rows of frames >= seq_len (no fbw_padfill in this call)
     int xs_cap = 0;              // general instance: edges its staging area holds beyond COMB_XS (0: no more)
-    int strips = 0;              // > 0: sequences of up to that many strips have rows of fbw_strips, with
+    int strips = 0;              // > 0: where fbw_strips takes the batch, sequences have rows of that kernel (or, overlapped, nothing is to do here), with
     const double* soffs = nullptr;   // an offset per direction, strip and block of frames (+inf: not walked), and
     const int* sprog = nullptr;      // a mark where they could not be computed (strip_lost)
+    int strips_only = 0;         // behind the kernels of the overlapped schedule: nothing to do unless fbw_strips has taken the batch
     int batch_frames = 0;        // SMALL instance: the LDS of the launch holds COMB_BATCH row images and staging areas (comb_batch_lds_bytes)
 };
+
+// Is the batch the other schedule's?  (Asked only where there are two.)
+template <bool SYNC>
+__device__ __forceinline__ bool comb_elsewhere(const CombArgs& a) {
+    return SYNC ? a.strips > 0 && a.sync[SYNC_UNCOVERED] == 0 : a.strips_only != 0 && a.sync[SYNC_UNCOVERED] != 0;
+}
 
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float float4a __attribute__((ext_vector_type(4)));
@@ -1971,7 +2000,7 @@ struct StripView {
     bool lost;                     // the rows could not be computed
 };
 __device__ __forceinline__ bool strip_view(StripView& v, const CombArgs& a, const SeqMeta& m, const int b, const int q) {
-    const int n = a.strips > 0 ? strip_count(m, b, a.T, a.strips) : 0;
+    const int n = a.strips > 0 ? strip_count(m, a.sync[SYNC_UNCOVERED] == 0) : 0;
     if (n == 0) return false;
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x, nblkT = (a.T + STRIP_FRAMES - 1) / STRIP_FRAMES;
@@ -2281,6 +2310,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
     const int tid = threadIdx.x;
     int b, y;
     strip_index(a.B, &b, &y);
+    if (comb_elsewhere<SYNC>(a)) return;
     const SeqMeta m = a.meta[b];
     if (!SMALL && a.pad_rows) {
         // Stage after stage there is nothing for fbw_padfill to run beside: its rows -- frames >= seq_len, for
@@ -3397,6 +3427,7 @@ __global__ __launch_bounds__(COMB_THREADS, NEGLOG ? (I6_FLAT_OCC < 6 ? I6_FLAT_O
     __shared__ int s_kind[12 * FLAT_KMAX];
     __shared__ long long s_off[4 * FLAT_KMAX];
     static_assert(FLAT_W >= COMB_FAST_EDGES, "the staging area of a posterior job lies in the image");
+    if (comb_elsewhere<SYNC>(fa.c)) return;
     const int B = fa.c.B, T = fa.c.T;
     const int n = (T + TC - 1) / TC;
     // job of this workgroup
@@ -3840,11 +3871,9 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // for CTC, whose last strip has edges of any kind (540 ns).  The device decides sequence by sequence (strip_count); here
     // only whether any of them can be meant.
     const bool strips_large = (long long)E > 1100LL * B;
-    const bool strips_pay = T >= 256 && (100LL * E <= 205LL * n_states || (strips_large && 10LL * E <= 23LL * n_states));
-    int strips = strips_pay && !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strips_to_launch(B, E, n_states) : 0;
-    const int strip_waves = strips;
-    if (strips > 0) strips |= (strips_large ? STRIPS_LARGE : STRIPS_CHAINS) << 8;
-    if (strips > 0 && strips_large && big && forced < 0) overlap = false;
+    const int strip_density = strips_large ? 230 : 205;
+    const bool strips_pay = T >= 256 && 100LL * E <= (long long)strip_density * n_states;
+    int strips = strips_pay && !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strips_to_launch(B, strip_states(B, E)) : 0;
     // All 2B recursion workgroups must be on the machine at the same time (at most two per compute
     // unit): gather and dense write wait for their progress while occupying wave slots themselves.
     if (2 * B > (dense ? 2 : 1) * P.n_cu) overlap = false;
@@ -3857,13 +3886,14 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // close it gets depends on its version.)
     if (dense && P.dense_regs > 104) overlap = false;
     // (a call that overlaps by its sizes keeps the same recursion, and the same bits, where capture or busy streams keep it from it)
-    if (overlap) strips = 0;
+    if (overlap && !(big && strips_large && forced < 0)) strips = 0;
     if (overlap) {
         // under stream capture: one stream, no in-memory waits between kernels, no synchronisation
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) overlap = false;
     }
     if (overlap) { int rc = runs_beside(P, s, &overlap); if (rc != I6FBW_OK) return rc; }
+    if (overlap && strips > 0) { int rc = runs_beside(P, P.sP, &overlap); if (rc != I6FBW_OK) return rc; }      // (see `both` below)
     hipStream_t sP = overlap ? P.sP : s, sR = overlap ? P.sR : s;
     const bool timed = g_prof.on && !static_call;     // stage timers create events
     if (timed) { std::lock_guard<std::mutex> plock(g_mutex); g_prof.n_calls++; }
@@ -3880,11 +3910,11 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     pa.ellA = (uint2*)(ws + l.ellA); pa.ellB = (uint2*)(ws + l.ellB);
     pa.crec = (uint4*)(ws + l.crec); pa.cbegin = (int*)(ws + l.cbegin); pa.demis = (int*)(ws + l.demis); pa.tband = (int2*)(ws + l.tband);
     pa.cflag = (int*)(ws + l.cflag); pa.wpfx = l.wpfx_stride > 0 ? (int*)(ws + l.wpfx) : nullptr; pa.wpfx_stride = l.wpfx_stride;
-    pa.strips = strips; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog);
+    pa.strips = strips; pa.strip_density = strip_density; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog);
     GatherArgs ga;
     ga.am = am; ga.st_t = am_stride_t; ga.st_b = am_stride_b; ga.T = T; ga.B = B;
     ga.meta = meta; ga.demis = pa.demis; ga.tband = pa.tband; ga.gtab = (float*)(ws + l.gtab); ga.sync = sync;
-    ga.scale = (input_flags & I6FBW_IN_LOG_PROBS) ? -LOG2E : LOG2E; ga.ascending = 0;
+    ga.scale = (input_flags & I6FBW_IN_LOG_PROBS) ? -LOG2E : LOG2E; ga.ascending = 0; ga.strips = overlap ? strips : 0;
     GenArgs gen;
     gen.am = am; gen.st_t = am_stride_t; gen.st_b = am_stride_b; gen.sign = (input_flags & I6FBW_IN_LOG_PROBS) ? -1.f : 1.f;
     gen.edges = edges; gen.edge_stride = edge_row_stride; gen.weights = weights; gen.eidx = pa.eidx; gen.renum = pa.renum;
@@ -3903,9 +3933,8 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     ca.out = out; ca.sum_output = sum_output; ca.ost_t = out_stride_t; ca.ost_b = out_stride_b; ca.sync = sync;
     ca.tile_w = tiled ? COMB_TILE_W : 0;
     ca.direct_only = 0;
-    wide = wide && !overlap;
-    if (wide) comb_lds += (size_t)(COMB_WIDE_EDGES - COMB_XS + COMB_MID_SLOTS) * 4;
-    ca.xs_cap = wide ? COMB_WIDE_EDGES : 0;
+    // (the stage-after-stage instance; in the overlapped schedule it is launched for the strips alone, behind the others)
+    const size_t wide_lds = comb_lds + (wide ? (size_t)(COMB_WIDE_EDGES - COMB_XS + COMB_MID_SLOTS) * 4 : 0);
     ca.strips = strips; ca.soffs = (const double*)(ws + l.soffs); ca.sprog = (const int*)(ws + l.sprog);
     // The dense tensor goes out in flat spans (fbw_flat) if it is one contiguous block in either
     // order of frames and sequences, rows are long enough for a span to cut at most two of them,
@@ -3917,7 +3946,8 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     bool flat = (writer > 0 || (writer < 0 && (overlap || (long long)T * B * F >= (1LL << 26)))) && flat_layout >= 0 &&
                 F >= FLAT_MIN_F && l.wpfx_stride > 0;
     FlatArgs fa;
-    long long flat_grid = 0;
+    long long flat_jobs = 0;
+    auto flat_grid = [&](const FlatArgs& f) { return dim3((unsigned)((long long)f.ahead * B * (TC / FLAT_TCF) + flat_jobs)); };
     if (flat) {
         const long long n = (T + TC - 1) / TC, rows = flat_layout == 0 ? B : 1;
         fa.c = ca; fa.layout = flat_layout;
@@ -3927,7 +3957,8 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
         fa.cflag = (int*)(ws + l.cflag); fa.wpfx = (const int*)(ws + l.wpfx); fa.wpfx_stride = l.wpfx_stride;
         fa.cp = ga.gtab;
         fa.ahead = overlap ? FLAT_AHEAD : FLAT_AHEAD_ALONE;
-        flat_grid = (long long)fa.ahead * B * (TC / FLAT_TCF) + (flat_layout == 0 ? n : n * B) * (fa.nW + rows * (TC / FLAT_TCF));
+        flat_jobs = (flat_layout == 0 ? n : n * B) * (fa.nW + rows * (TC / FLAT_TCF));
+        const long long flat_grid = (long long)std::max(FLAT_AHEAD, FLAT_AHEAD_ALONE) * B * (TC / FLAT_TCF) + flat_jobs;
         if (flat_grid > 0x7fffffffLL || (long long)TC * rows * F >= (1LL << 31) - FLAT_W) flat = false;
     }
     ca.direct_only = flat ? 1 : 0;
@@ -3943,7 +3974,10 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // Where the recursion kernel is started: beside the preparation if its 2B workgroups leave at
     // least half of the compute units empty (the preparation's workgroups need most of a unit's
     // LDS and could otherwise find no room while the recursion waits for them), else behind it.
-    const bool early = overlap && 2 * B <= P.n_cu / 2;
+    // (not where the strips may take the batch, see below: there the streams part behind the preparation, at a single event on the
+    // caller's, which holds it up for some ten microseconds)
+    const bool both = overlap && strips > 0;
+    const bool early = overlap && !both && 2 * B <= P.n_cu / 2;
     // The preparation's workgroups can do the gate's wait themselves (one kernel less in front of the gather)
     // where they cannot be in the recursion's way: a preparation workgroup and a recursion workgroup do not
     // share a compute unit, the order in which the two kernels are placed is not ours, and a preparation
@@ -3982,8 +4016,10 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
         // slots on one compute unit each and find them while the machine is still almost empty;
         // they wait in memory for the preparation to finish (fbw_prepare counts its workgroups),
         // and their loader waves later for the gather's strip flags.
-        HIP_TRY(hipEventRecord(P.start, s));
-        HIP_TRY(hipStreamWaitEvent(sP, P.start, 0));
+        if (!both) {
+            HIP_TRY(hipEventRecord(P.start, s));
+            HIP_TRY(hipStreamWaitEvent(sP, P.start, 0));
+        }
         if (early) {
             HIP_TRY(hipStreamWaitEvent(sR, P.start, 0));
             int rc = launch_recursion(); if (rc != I6FBW_OK) return rc;
@@ -4000,8 +4036,8 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
         int rc = launch_recursion(); if (rc != I6FBW_OK) return rc;
     }
     // (with the flat writer, the row writer for the sequences fbw_flat leaves out is started below, behind the gather)
-    ca.pad_rows = (!flat && !overlap) ? 1 : 0;
-    if (!flat && overlap) {
+    ca.pad_rows = (!flat && (!overlap || strips > 0)) ? 1 : 0;
+    if (!flat && overlap && strips == 0) {
         // Rows of frames beyond seq_len depend on seq_lens only: written beside the preparation, which
         // leaves the memory system idle.  (Stage after stage the row writer takes them, see pad_rows.)
         StageTimer tm(4, sP, timed);
@@ -4011,18 +4047,35 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     }
     if (overlap) HIP_TRY(hipEventRecord(P.doneP, sP));
 
+    // Gather and recursion over strips, for batches that can be cut that way (the kernels find that out by themselves).
+    auto launch_strips = [&](hipStream_t st) -> int {
+        StripGatherArgs sg;
+        sg.g = ga; sg.ell = pa.ellA; sg.etab = (float*)(ws + l.etab); sg.strips = strips; sg.cap = strip_gather_lds(B, E); sg.keep_rows = 1; sg.soffs = (double*)(ws + l.soffs);
+        sg.strips_only = overlap ? 1 : 0;
+        FbwStripArgs sa;
+        sa.T = T; sa.B = B; sa.strips = strips; sa.meta = meta; sa.ellA = pa.ellA; sa.ellB = pa.ellB; sa.gtab = ga.gtab; sa.etab = sg.etab;
+        sa.alpha = ra.alpha; sa.beta = ra.beta; sa.soffs = sg.soffs; sa.halo = (double*)(ws + l.shalo); sa.prog = pa.sprog; sa.sync = sync;
+        { StageTimer tm(1, st, timed); hipLaunchKernelGGL(strip_gather, g_grid, dim3(256), sg.cap * sizeof(float), st, sg); }
+        HIP_TRY(hipGetLastError());
+        StageTimer tm(2, st, timed);
+        hipLaunchKernelGGL(fbw_strips, dim3((unsigned)(2 * B * ((strips + STRIP_WAVES - 1) / STRIP_WAVES))), dim3(STRIP_BLOCK), 0, st, sa);
+        HIP_TRY(hipGetLastError());
+        return I6FBW_OK;
+    };
+    auto launch_rows = [&](hipStream_t st, CombArgs c, FlatArgs f) -> int {
+        c.xs_cap = wide ? COMB_WIDE_EDGES : 0;
+        f.c = c; f.ahead = FLAT_AHEAD_ALONE;
+        if (flat) {
+            // (the row kernel first: it only has the sequences that are too large for the other one)
+            { StageTimer tm(4, st, timed); launch_combine<false>(neglog, c_grid, wide_lds, st, c); }
+            { StageTimer tm(3, st, timed); launch_flat<false>(neglog, flat_grid(f), st, f); }
+        } else { StageTimer tm(3, st, timed); launch_combine<false>(neglog, c_grid, wide_lds, st, c); }
+        HIP_TRY(hipGetLastError());
+        return I6FBW_OK;
+    };
     if (!overlap) {
-        if (strips > 0) {
-            StripGatherArgs sg;
-            sg.g = ga; sg.ell = pa.ellA; sg.etab = (float*)(ws + l.etab); sg.strips = strips; sg.cap = strip_gather_lds(B, E); sg.keep_rows = 1; sg.soffs = (double*)(ws + l.soffs);
-            FbwStripArgs sa;
-            sa.T = T; sa.B = B; sa.strips = strips; sa.meta = meta; sa.ellA = pa.ellA; sa.ellB = pa.ellB; sa.gtab = ga.gtab; sa.etab = sg.etab;
-            sa.alpha = ra.alpha; sa.beta = ra.beta; sa.soffs = sg.soffs; sa.halo = (double*)(ws + l.shalo); sa.prog = pa.sprog; sa.sync = sync;
-            { StageTimer tm(1, s, timed); hipLaunchKernelGGL(strip_gather, g_grid, dim3(256), sg.cap * sizeof(float), s, sg); }
-            HIP_TRY(hipGetLastError());
-            StageTimer tm(2, s, timed);
-            hipLaunchKernelGGL(fbw_strips, dim3((unsigned)(2 * B * ((strip_waves + STRIP_WAVES - 1) / STRIP_WAVES))), dim3(STRIP_BLOCK), 0, s, sa);
-        } else {
+        if (strips > 0) { int rc = launch_strips(s); if (rc != I6FBW_OK) return rc; }
+        else {
             StageTimer tm(1, s, timed);
             hipLaunchKernelGGL(fbw_gather<false>, g_grid, dim3(256), 0, s, ga);
         }
@@ -4031,51 +4084,66 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
           else if (big) hipLaunchKernelGGL(fbw_recurse_big<false>, dim3(2 * B), dim3(REC_BLOCK_BIG), 0, s, ra);
           else hipLaunchKernelGGL(fbw_recurse<false>, dim3(2 * B), dim3(REC_BLOCK), 0, s, ra); }
         HIP_TRY(hipGetLastError());
-        if (flat) {
-            // (the row kernel first: it only has the sequences that are too large for the other one)
-            { StageTimer tm(4, s, timed); launch_combine<false>(neglog, c_grid, comb_lds, s, ca); }
-            { StageTimer tm(3, s, timed); launch_flat<false>(neglog, dim3((unsigned)flat_grid), s, fa); }
-        } else { StageTimer tm(3, s, timed); launch_combine<false>(neglog, c_grid, comb_lds, s, ca); }
-        HIP_TRY(hipGetLastError());
-        return I6FBW_OK;
+        return launch_rows(s, ca, fa);
     }
 
+    // Large automata (strips > 0): only the preparation can tell whether the strips can take the batch.  Where they can, they need 1190 us
+    // for what the overlapped stages need 1960 (8 sequences of 1750 states, T=2500 F=5000); where they cannot -- an edge five
+    // states upward, say -- those stages are 1.2 to 1.4 times as fast as the same kernels one after the other.  So both are
+    // enqueued, and the one whose turn it is not ends at once: the strips on the caller's stream, gather and dense write of the
+    // overlapped schedule on the library's.  (Batches for the strips pay 1 to 2 % for it: an event, the other kernels' workgroups.)
+    hipStream_t sG = both ? sP : s, sD = both ? s : sP;        // gather and dense write; the rows that fbw_flat leaves out
+    // (tens of thousands of workgroups for batches that the strips take, and little more than holes for automata of that size)
+    const bool spans = flat && !(both && (long long)E > (long long)FLAT_EDGES * B);
+    CombArgs co = ca;
+    if (flat && !spans) { co.direct_only = 0; co.pad_rows = 1; }
+    if (both) {
+        HIP_TRY(hipStreamWaitEvent(sG, P.fork, 0));
+        CombArgs cs = ca;
+        cs.strips_only = 1;
+        { int rc = launch_strips(s); if (rc != I6FBW_OK) return rc; }
+        { int rc = launch_rows(s, cs, fa); if (rc != I6FBW_OK) return rc; }
+    }
     // A running grid of small workgroups refills every wave slot it frees, so gather and dense
     // write (which also wait for recursion progress while they occupy LDS and wave slots) are
     // held back until every recursion workgroup is on the machine -- normally long since.
     // (Or by the preparation's workgroups at their end, see gate_in_prepare.)
     if (!gate_in_prepare) {
-        hipLaunchKernelGGL(fbw_gate, dim3(1), dim3(64), 0, s, sync, 2 * B);
+        hipLaunchKernelGGL(fbw_gate, dim3(1), dim3(64), 0, sG, sync, 2 * B);
         HIP_TRY(hipGetLastError());
     }
-    { StageTimer tm(1, s, timed); hipLaunchKernelGGL(fbw_gather<true>, g_grid, dim3(256), 0, s, ga); }
+    { StageTimer tm(1, sG, timed); hipLaunchKernelGGL(fbw_gather<true>, g_grid, dim3(256), 0, sG, ga); }
     HIP_TRY(hipGetLastError());
-    if (flat) {
+    if (spans) {
         // fbw_flat writes every row except those of sequences too large for its posterior jobs: these go
-        // row by row through fbw_combine on the second library stream, beside fbw_flat (the two kernels
+        // row by row through fbw_combine on another stream, beside fbw_flat (the two kernels
         // do not wait for each other).  It is started behind the gather like fbw_flat itself: its
         // workgroups wait for the gather's strips while they hold registers and wave slots, so they
         // must not be on the machine before the gather's own are (three of them fill a compute unit's
         // register file).  It has nothing to do for the usual batch.
-        HIP_TRY(hipEventRecord(P.gathered, s));
-        HIP_TRY(hipStreamWaitEvent(sP, P.gathered, 0));
-        { StageTimer tm(4, sP, timed); launch_combine<true>(neglog, c_grid, comb_lds, sP, ca); }
+        HIP_TRY(hipEventRecord(P.gathered, sG));
+        HIP_TRY(hipStreamWaitEvent(sD, P.gathered, 0));
+        { StageTimer tm(4, sD, timed); launch_combine<true>(neglog, c_grid, comb_lds, sD, ca); }
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipEventRecord(P.doneP, sP));
+        if (!both) HIP_TRY(hipEventRecord(P.doneP, sP));
     }
     // The dense write follows the gather on the same stream (its workgroups would only take wave
     // slots away from the gather before that: by then the two recursions are about to meet in the
     // middle of the sequences, where the dense write begins); each of its workgroups waits for the
     // recursion progress it needs.
 #ifdef I6_TRACE
-    if (getenv("I6FBW_DBG_SERIAL_COMBINE")) HIP_TRY(hipStreamWaitEvent(s, P.doneR, 0));
+    if (getenv("I6FBW_DBG_SERIAL_COMBINE")) HIP_TRY(hipStreamWaitEvent(sG, P.doneR, 0));
 #endif
-    if (flat) { StageTimer tm(3, s, timed); launch_flat<true>(neglog, dim3((unsigned)flat_grid), s, fa); }
-    else { StageTimer tm(3, s, timed); launch_combine<true>(neglog, c_grid, comb_lds, s, ca); }
+    if (spans) { StageTimer tm(3, sG, timed); launch_flat<true>(neglog, flat_grid(fa), sG, fa); }
+    else { StageTimer tm(3, sG, timed); launch_combine<true>(neglog, c_grid, comb_lds, sG, co); }
     HIP_TRY(hipGetLastError());
+    if (both) {
+        HIP_TRY(hipStreamWaitEvent(sP, P.doneR, 0));
+        HIP_TRY(hipEventRecord(P.doneP, sP));
+    }
     // join: both finish well before the dense write does
     HIP_TRY(hipStreamWaitEvent(s, P.doneP, 0));
-    HIP_TRY(hipStreamWaitEvent(s, P.doneR, 0));
+    if (!both) HIP_TRY(hipStreamWaitEvent(s, P.doneR, 0));
     join_guard.joined = true;
     return I6FBW_OK;
 }

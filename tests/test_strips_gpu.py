@@ -21,7 +21,7 @@ def stage_after_stage():
 def automata(rng, sizes, F, kind, permute=False):
     """Left-to-right automata of the given numbers of states.  kind: "chain" loops and steps; "optional" some states can be
     passed over; "ctc" emission on the target state and several edges into the last state; "wide" edges of up to four
-    states upward, some of them twice; "far" one edge of five (not for the strips).  Weights are multiples of 1/2, so ties are common."""
+    states upward, some of them twice; "far" one edge of five (not for the strips); "mixed" that in the last sequence only.  Weights are multiples of 1/2, so ties are common."""
     frm, to, emis, seq, w = [], [], [], [], []
     ends = []
     off = 0
@@ -39,7 +39,7 @@ def automata(rng, sizes, F, kind, permute=False):
                 steps.append(2)
             if kind == "wide":
                 steps += [int(x) for x in rng.integers(1, 5, size=rng.integers(0, 2))]
-            if kind == "far" and u == n // 3:
+            if (kind == "far" or (kind == "mixed" and b == len(sizes) - 1)) and u == n // 3:
                 steps.append(5)
             for k in steps:
                 if u + k < n and not (kind == "ctc" and u + k == n - 1 and k == 0):
@@ -71,6 +71,7 @@ CASES = [
     ([6, 61, 125, 242, 300], 330, [330, 200, 329, 328, 327], 60, "ctc"),                         # strips with edges of any kind
     ([70, 130, 250, 64], 180, [180, 179, 177, 64], 31, "wide"),
     ([70, 130, 250, 64], 280, [280, 279, 277, 64], 31, "far"),                                   # the other kernels
+    ([70, 130, 250, 64], 280, [280, 279, 277, 64], 31, "mixed"),                                 # for the whole batch
     ([300, 200, 100], 150, [150, 100, 99], 50, "chain"),                                         # the end is out of reach for two of them
     ([1900, 1100], 2304, [2301, 1100], 700, "optional"),                                         # many workgroups, several passes of the gather
 ]
@@ -234,3 +235,74 @@ def test_best_path_waits_that_run_out(oracle):
         else:
             assert_identical((align[:, b], scores[b:b + 1]), (want[0][:, b], want[1][b:b + 1]))
     assert_identical(run_cabi_viterbi(*args)[:2], want)
+
+
+def run_without_strips(am, edges, weights, start_end, seq_lens, n_states, out_mode):
+    """The same call in a workspace that ends before the strips' tables."""
+    from tests.gpu_util import DeviceProblem
+    P = DeviceProblem(am, edges, weights, start_end, seq_lens, n_states)
+    P.ws_bytes -= 256
+    out, loss = P.run(out_mode)
+    return out.cpu().numpy(), loss.cpu().numpy()
+
+
+@pytest.mark.parametrize("kind", ["chain", "mixed"])
+def test_a_batch_goes_through_the_strips_as_a_whole(oracle, kind):
+    """One sequence that they cannot take, and the others go with it: the two recursions one behind the other would take as
+    long as both.  (Seen by the bits, which are those of a call without strips then.)"""
+    from tests.gpu_util import run_cabi
+    from tests.helpers import posterior
+    rng = np.random.default_rng(21)
+    edges, weights, start_end, n = automata(rng, [200, 250, 190], 40, kind)
+    am = rng.uniform(0.1, 9.0, size=(420, 3, 40)).astype(np.float32)
+    args = (am, edges, -weights, start_end, np.array([420, 411, 300], dtype=np.int32), n)
+    out, loss = run_cabi(*args, out_mode=cabi.OUT_PROB)
+    want_out, want_loss = oracle.fbw_oracle(*args, threads=4)
+    np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(out, posterior(want_out), rtol=0, atol=1e-4)
+    other, _ = run_without_strips(*args, cabi.OUT_PROB)
+    assert np.array_equal(out, other) == (kind == "mixed")
+
+
+@pytest.mark.parametrize("writer", [0, 1], ids=["rows", "flat"])
+@pytest.mark.parametrize("kind", ["optional", "mixed"])
+def test_large_automata_overlapped_or_in_strips(oracle, kind, writer):
+    """Calls whose sizes ask for the overlapped schedule: enqueued both ways, the preparation decides."""
+    from tests.gpu_util import run_cabi
+    from tests.helpers import posterior
+    rng = np.random.default_rng(22)
+    T, B, F = 1025, 5, 13100
+    assert T * B * F >= 1 << 26
+    edges, weights, start_end, n = automata(rng, rng.integers(590, 650, size=B).tolist(), F, kind)
+    # (few states can be passed over: 2.3 edges per state is the limit for automata of this size)
+    keep = (edges[1] - edges[0] != 2) | (rng.random(edges.shape[1]) < 0.4)
+    edges, weights = edges[:, keep].copy(), weights[keep].copy()
+    am = rng.uniform(0.1, 9.0, size=(T, B, F)).astype(np.float32)
+    lens = rng.integers(660, T + 1, size=B).astype(np.int32)
+    lens[1] = T
+    args = (am, edges, -weights, start_end, lens, n)
+    want_out, want_loss = oracle.fbw_oracle(*args, threads=8)
+    cabi.set_dense_writer(writer)
+    try:
+        cabi.set_overlap(-1)
+        out, loss = run_cabi(*args, out_mode=cabi.OUT_PROB)
+        cabi.set_overlap(1)         # (leaves the strips out)
+        overlapped, _ = run_cabi(*args, out_mode=cabi.OUT_PROB)
+    finally:
+        cabi.set_dense_writer(-1)
+    np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(out, posterior(want_out), rtol=0, atol=1e-4)
+    assert np.array_equal(out, overlapped) == (kind == "mixed")
+
+
+@pytest.mark.parametrize("kind", ["optional", "mixed", "far"])
+def test_best_path_overlapped_or_in_strips(oracle, kind):
+    rng = np.random.default_rng(23)
+    T, B, F = 800, 13, 6500
+    assert T * B * F >= 1 << 26
+    cabi.set_overlap(-1)
+    edges, weights, start_end, n = automata(rng, rng.integers(60, 200, size=B).tolist(), F, kind, permute=True)
+    am = -0.25 * rng.integers(0, 12, size=(T, B, F)).astype(np.float32)
+    args = (am, edges, weights, start_end, rng.integers(300, T + 1, size=B).astype(np.int32), n)
+    for rep in range(2):
+        assert_identical(run_cabi_viterbi(*args)[:2], oracle.viterbi_oracle(*args))
