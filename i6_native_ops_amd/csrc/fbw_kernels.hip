@@ -312,6 +312,37 @@ inline int strips_to_launch(const int B, const long long average_states) {
 }
 // The average in a full sum over strips, where the automata have about two edges per state, from the edges alone: see strip_density
 inline long long strip_states(const int B, const int E) { return ((long long)E + B) / (2LL * B) + 1; }
+inline long long strip_groups(const long long states) { return (strips_of((int)std::min(states, (long long)S_MAX)) + 3) / 4; }
+
+// Full sum: up to how many edges per 100 states the strips pay, 0 where they do not.  A workgroup of fbw_strips, four strips in one
+// direction, takes a compute unit to itself (211 registers): once there are more of them than units they run in rounds, where the
+// other recursion has one workgroup per sequence and direction.  Call with strips / without (T frames, F = 200-264; n: workgroups):
+//   chains, 60 states, T=300:     1.07 at B=1, 0.97 from 16 to 64, 1.07 from 128 on; 100-180 states 0.94-0.96 up to 64, 1.00 at 96,
+//                                 1.03 from 128 on; over 500-1000 frames 180-240 states 0.80-0.95 up to 128, 1.07 at 192
+//   375 states, T=1000:           0.74 ... 0.94 at n=256, 1.12 at 384
+//   500 and 560 states, T=1000:   0.57 ... 0.85 and 0.97 at n=576, 0.92 and 1.01 at 768;  900-1750 states: 0.42 ... 0.83 at 1024
+//   2.14 edges per state, 375 states: 0.79 ... 1.05 at n=256, but 180 states 1.02 at n=64 (strip_gather writes three scores per state);
+//   560 states 0.89 at n=192, 1.09 at 384; 900 0.86 at 256, 0.98 at 512; 1300-1750 0.84 at 384-512, 1.05 at 768-1024
+//   2.6 edges per state: as with 2.14 -- the line is at 2.3 because CTC automata have 2.5 less their repeated labels: with the
+//   edges into their last state a wave takes 540 ns a frame (301 states 1.27-1.34, 601 states 0.99-1.24)
+inline int strip_density(const int T, const int B, const int E, const int n_cu) {
+    if (T < 256) return 0;
+    const long long states = strip_states(B, E), n = 2LL * B * strip_groups(states);
+    if ((long long)E > 1100LL * B && n <= (states > 1024 ? 2LL : 1LL) * n_cu) return 230;
+    const long long most = states < 96 ? 0 : states <= 480 ? (states > 256 ? n_cu : T >= 384 ? n_cu / 2 : n_cu / 4) : (states > 720 ? 4LL : 2LL) * n_cu;
+    return n <= most ? 205 : 0;
+}
+// Best path: the same question.  Call with strips / without: chains and 2.14 edges per state, 60-180 states 0.62 ... 0.95 and 0.99 at n=256;
+// 375 states 0.60 ... 0.86 at n=256, 0.99 at 384, 1.11 at 512; 900 states 0.43 ... 0.70 at 768; 1750 states 0.27 ... 0.87 at 768, 1.16
+// at 1024.  More than 2.4 edges per state (CTC, whose last strip has edges of any kind, or all strips of that kind): 81 states
+// 0.95 up to n=64, 1.02 at 96, 1.07 at 128; 201 and 401 states 0.77 ... 0.86-0.99 at 64, 1.02-1.05 at 128; 551-851 states 0.50 ... 0.80 at 256,
+// 1.02 at 384; 1001 states 0.46 ... 0.53 at 1280 (more than 1024 states of that degree: 3.4 us a frame in the search);
+// five edges per state, 375 states: 0.95 up to 32, 1.01 at 64, 1.5 beyond 256; and slower than the search beside the gather (1.09).
+inline bool best_path_strips(const int B, const int E, const int n_states, const int n_cu, const bool overlap) {
+    const long long states = std::min((long long)n_states, (long long)E + B) / B + 1, n = B * strip_groups(states);
+    if (10LL * E > 24LL * n_states) return !overlap && n <= (states > 1024 ? 4LL * n_cu : states > 512 ? n_cu : n_cu / 4);
+    return n <= (states > 512 ? 3LL : 1LL) * n_cu;
+}
 
 // Hand-off between kernels that run at the same time (gather -> recursion -> combine).  The
 // L2 caches of the eight XCDs are not coherent with each other inside a kernel, so everything
@@ -789,6 +820,11 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
                 }
                 __syncthreads();
             }
+            // (on a cycle the hops double to more than there are states: no heights, and nothing to wait for in the other picks --
+            // 2 to 26 % of a best-path call)
+            int cyclic = 0;
+            for (int r = tid; r < nS; r += NT) cyclic |= (int)(dn[r] >> 16) >= nS;
+            if (__syncthreads_or(cyclic)) break;
         }
         if (!rest) by_level = false;
         else {
@@ -3866,14 +3902,10 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
                                : ((long long)T * B * F >= (1LL << 26) && 2 * B <= P.n_cu / 2 && T >= 384 && (B >= 12 || T >= 1000));
     // The strip kernels take the place of the recursion stage after stage: also where the overlap would pay for the large
     // instance.  (The dump of the forward scores reads rows in the layout of the other kernels.)
-    // They pay for chains (two candidates per state: 115 ns a frame where fbw_recurse takes 170) and for large automata with
-    // optional states (180 instead of 680), not for small ones with three candidates (172 / 196 ns, but a larger gather) nor
-    // for CTC, whose last strip has edges of any kind (540 ns).  The device decides sequence by sequence (strip_count); here
-    // only whether any of them can be meant.
+    // (strip_density says where they pay; whether all sequences are such automata is found out by the preparation)
     const bool strips_large = (long long)E > 1100LL * B;
-    const int strip_density = strips_large ? 230 : 205;
-    const bool strips_pay = T >= 256 && 100LL * E <= (long long)strip_density * n_states;
-    int strips = strips_pay && !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strips_to_launch(B, strip_states(B, E)) : 0;
+    const int density = !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strip_density(T, B, E, P.n_cu) : 0;
+    int strips = density > 0 && 100LL * E <= (long long)density * n_states ? strips_to_launch(B, strip_states(B, E)) : 0;
     // All 2B recursion workgroups must be on the machine at the same time (at most two per compute
     // unit): gather and dense write wait for their progress while occupying wave slots themselves.
     if (2 * B > (dense ? 2 : 1) * P.n_cu) overlap = false;
@@ -3910,7 +3942,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     pa.ellA = (uint2*)(ws + l.ellA); pa.ellB = (uint2*)(ws + l.ellB);
     pa.crec = (uint4*)(ws + l.crec); pa.cbegin = (int*)(ws + l.cbegin); pa.demis = (int*)(ws + l.demis); pa.tband = (int2*)(ws + l.tband);
     pa.cflag = (int*)(ws + l.cflag); pa.wpfx = l.wpfx_stride > 0 ? (int*)(ws + l.wpfx) : nullptr; pa.wpfx_stride = l.wpfx_stride;
-    pa.strips = strips; pa.strip_density = strip_density; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog);
+    pa.strips = strips; pa.strip_density = density; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog);
     GatherArgs ga;
     ga.am = am; ga.st_t = am_stride_t; ga.st_b = am_stride_b; ga.T = T; ga.B = B;
     ga.meta = meta; ga.demis = pa.demis; ga.tband = pa.tband; ga.gtab = (float*)(ws + l.gtab); ga.sync = sync;

@@ -21,7 +21,9 @@ def stage_after_stage():
 def automata(rng, sizes, F, kind, permute=False):
     """Left-to-right automata of the given numbers of states.  kind: "chain" loops and steps; "optional" some states can be
     passed over; "ctc" emission on the target state and several edges into the last state; "wide" edges of up to four
-    states upward, some of them twice; "far" one edge of five (not for the strips); "mixed" that in the last sequence only.  Weights are multiples of 1/2, so ties are common."""
+    states upward, some of them twice; "far" one edge of five (not for the strips); "mixed" that in the last sequence only;
+    "sparse" like wide, but few of those edges, and "passing" like optional, but few such states (2.05 and 2.3 edges per state at
+    most, what the full sum leaves to the strips).  Weights are multiples of 1/2, so ties are common."""
     frm, to, emis, seq, w = [], [], [], [], []
     ends = []
     off = 0
@@ -37,6 +39,10 @@ def automata(rng, sizes, F, kind, permute=False):
             steps = [0, 1]
             if kind in ("optional", "ctc") and rng.random() < 0.4:
                 steps.append(2)
+            if kind == "passing" and rng.random() < 0.2:
+                steps.append(2)
+            if kind == "sparse" and (u % 60 in (1, 56, 57) or u in (235, 236, 239)) and (u // 60) % 2 == 0:
+                steps.append(int(rng.choice([1, 3, 4, 2])))
             if kind == "wide":
                 steps += [int(x) for x in rng.integers(1, 5, size=rng.integers(0, 2))]
             if (kind == "far" or (kind == "mixed" and b == len(sizes) - 1)) and u == n // 3:
@@ -144,25 +150,140 @@ FULL_SUM = [
     ([119, 120, 121, 176, 180, 181], 264, [264, 263, 257, 256, 199, 264], 40, "chain"),      # borders of strips, of blocks, of the last block
     ([236, 240, 244, 480], 600, [600, 599, 593, 592], 97, "chain"),                          # borders of workgroups
     ([300, 290, 20], 304, [301, 290, 5], 50, "chain"),                                       # just enough frames; an end out of reach
-    ([700, 650, 1200], 1288, [1288, 1281, 1250], 300, "optional"),                           # large, three sources per state
+    ([700, 650, 1200], 1288, [1288, 1281, 1250], 300, "passing"),                            # large, three sources per state
+    ([180, 247, 300, 121], 304, [304, 303, 301, 297], 50, "sparse"),                         # strips with edges of any kind
+    ([700, 650, 1200], 808, [808, 801, 790], 300, "passing"),                                # the same, fewer frames than states
 ]
+
+
+def run_without_strips(am, edges, weights, start_end, seq_lens, n_states, out_mode):
+    """The same call in a workspace that ends before the strips' tables."""
+    from tests.gpu_util import DeviceProblem
+    P = DeviceProblem(am, edges, weights, start_end, seq_lens, n_states)
+    P.ws_bytes -= 256
+    out, loss = P.run(out_mode)
+    return out.cpu().numpy(), loss.cpu().numpy()
+
+
+def check_full_sum(oracle, args, strips=True):
+    """Both output modes; losses to 1e-5 and posteriors to 1e-4 of the oracle's, the bars of the other full-sum tests.  Other bits
+    than without strips show that the strips were there."""
+    from tests.gpu_util import run_cabi
+    from tests.helpers import posterior
+    want_out, want_loss = oracle.fbw_oracle(*args, threads=4)
+    out, loss = run_cabi(*args)
+    np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(posterior(out), posterior(want_out), rtol=0, atol=1e-4)
+    assert (np.isposinf(out) == np.isposinf(want_out)).all()
+    prob, loss = run_cabi(*args, out_mode=cabi.OUT_PROB)
+    np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(prob, posterior(want_out), rtol=0, atol=1e-4)
+    other, _ = run_without_strips(*args, cabi.OUT_PROB)
+    assert strips != np.array_equal(prob, other)
 
 
 @pytest.mark.parametrize("permute", [False, True], ids=["in_order", "permuted"])
 @pytest.mark.parametrize("case", range(len(FULL_SUM)))
 def test_full_sum(oracle, case, permute):
-    """Losses to 1e-5 and posteriors to 1e-4 of the oracle's, the bars of the other full-sum tests."""
-    from tests.gpu_util import run_cabi
-    from tests.helpers import posterior
     sizes, T, lens, F, kind = FULL_SUM[case]
     rng = np.random.default_rng(300 + case)
     edges, weights, start_end, n = automata(rng, sizes, F, kind, permute)
     am = rng.uniform(0.1, 9.0, size=(T, len(sizes), F)).astype(np.float32)
     args = (am, edges, -weights, start_end, np.array(lens, dtype=np.int32), n)
+    # (ids that do not follow a small automaton are only renumbered where it is tightly aligned, and its batch goes elsewhere then)
+    check_full_sum(oracle, args, strips=not (permute and case in (0, 1, 4)))
+
+
+def test_full_sum_over_impossible_scores(oracle):
+    """Scores of +inf (probability 0): scattered ones, a class that is never possible, a frame that lets nothing pass."""
+    rng = np.random.default_rng(31)
+    for kind, sizes, T in (("chain", [200, 130, 190], 424), ("passing", [700, 610, 660], 960)):
+        edges, weights, start_end, n = automata(rng, sizes, 60, kind)
+        am = rng.uniform(0.1, 9.0, size=(T, 3, 60)).astype(np.float32)
+        am[rng.random(am.shape) < 0.005] = np.inf      # (a chain over 60 classes finds no way through 0.02)
+        am[:, 1, 7] = np.inf
+        am[T // 2, 2, :] = np.inf
+        check_full_sum(oracle, (am, edges, -weights, start_end, np.array([T, T - 5, T - 9], dtype=np.int32), n))
+
+
+def test_full_sum_scores_that_are_not_numbers_stay_in_their_sequence(oracle):
+    """(What they make of their own sequence is not pinned: the reference skips some and loses the sequence over others.)"""
+    from tests.gpu_util import run_cabi
+    rng = np.random.default_rng(32)
+    for bad in (np.nan, -np.inf):
+        for kind, sizes, T in (("chain", [200, 130, 190], 424), ("passing", [700, 610, 660], 960)):
+            edges, weights, start_end, n = automata(rng, sizes, 60, kind)
+            am = rng.uniform(0.1, 9.0, size=(T, 3, 60)).astype(np.float32)
+            args = [am, edges, -weights, start_end, np.array([T, T - 5, T - 9], dtype=np.int32), n]
+            want, want_loss = run_cabi(*args, out_mode=cabi.OUT_PROB)
+            args[0] = am.copy()
+            args[0][:, 1][rng.random((T, 60)) < 0.01] = bad
+            out, loss = run_cabi(*args, out_mode=cabi.OUT_PROB)
+            for b in (0, 2):
+                np.testing.assert_array_equal(out[:, b], want[:, b])
+                np.testing.assert_array_equal(loss[:, b], want_loss[:, b])
+
+
+@pytest.mark.parametrize("n_edges", [4095, 4096, 4097, 4607, 4608, 4609])
+def test_row_writer_staging_area(oracle, n_edges):
+    """One automaton on both sides of what the row writer keeps in registers (4096 edges) and of what it stages at once (4608),
+    behind the strips and behind the other recursion; a small one beside it."""
+    from tests.helpers import posterior
+    rng = np.random.default_rng(n_edges)
+    S, T = 2040, 2304
+    edges, weights, start_end, n = automata(rng, [S, 30], 700, "optional")
+    frm, to, emis, seq = edges
+    spare = np.flatnonzero((seq == 0) & (to - frm == 2))            # states that can be passed over: as many as it takes
+    drop = int((seq == 0).sum()) - n_edges
+    assert 0 <= drop <= spare.size
+    keep = np.ones(edges.shape[1], dtype=bool)
+    keep[spare[:drop]] = False
+    keep[(seq == 1) & (to - frm == 2)] = False          # (the small one a chain: more than 2.3 edges per state would keep the strips out)
+    edges, weights = edges[:, keep].copy(), weights[keep].copy()
+    assert (edges[3] == 0).sum() == n_edges
+    am = rng.uniform(0.1, 9.0, size=(T, 2, 700)).astype(np.float32)
+    args = (am, edges, -weights, start_end, np.array([2301, 300], dtype=np.int32), n)
+    check_full_sum(oracle, args, strips=n_edges <= 23 * S // 10)
+    other, loss = run_without_strips(*args, cabi.OUT_PROB)
     want_out, want_loss = oracle.fbw_oracle(*args, threads=4)
-    out, loss = run_cabi(*args)
     np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
-    np.testing.assert_allclose(posterior(out), posterior(want_out), rtol=0, atol=1e-4)
+    np.testing.assert_allclose(other, posterior(want_out), rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("B", [16, 160])
+def test_batches_with_more_strips_than_compute_units(oracle, B):
+    """The full sum leaves them to the other recursion, which needs no second round of workgroups (same bits as without strips)."""
+    rng = np.random.default_rng(B)
+    edges, weights, start_end, n = automata(rng, rng.integers(120, 200, size=B).tolist(), 20, "chain")
+    am = rng.uniform(0.1, 9.0, size=(256, B, 20)).astype(np.float32)
+    check_full_sum(oracle, (am, edges, -weights, start_end, rng.integers(210, 257, size=B).astype(np.int32), n), strips=B == 16)
+
+
+def test_replayed_graph_of_the_full_sum(oracle):
+    """Progress counters, marks and offsets start afresh on every replay of a captured call."""
+    from tests.gpu_util import DeviceProblem
+    from tests.helpers import posterior
+    rng = np.random.default_rng(12)
+    edges, weights, start_end, n = automata(rng, [300, 250], 40, "chain")
+    seq_lens = np.array([420, 400], dtype=np.int32)
+    am = rng.uniform(0.1, 9.0, size=(420, 2, 40)).astype(np.float32)
+    P = DeviceProblem(am, edges, -weights, start_end, seq_lens, n)
+    P.run(cabi.OUT_PROB)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        P.run(cabi.OUT_PROB, check=False)
+    for i in range(4):
+        am = rng.uniform(0.1, 9.0, size=am.shape).astype(np.float32)
+        P.am.copy_(torch.from_numpy(am))
+        P.out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        out, loss = P.out.cpu().numpy().copy(), P.loss.cpu().numpy().copy()
+        want_out, want_loss = oracle.fbw_oracle(am, edges, -weights, start_end, seq_lens, n, threads=4)
+        np.testing.assert_allclose(loss, want_loss, rtol=1e-5, atol=1e-6)
+        np.testing.assert_allclose(out, posterior(want_out), rtol=0, atol=1e-4)
+        eager, _ = P.run(cabi.OUT_PROB)
+        np.testing.assert_array_equal(out, eager.cpu().numpy())
 
 
 def test_last_block_of_a_tight_sequence(oracle):
@@ -237,15 +358,6 @@ def test_best_path_waits_that_run_out(oracle):
     assert_identical(run_cabi_viterbi(*args)[:2], want)
 
 
-def run_without_strips(am, edges, weights, start_end, seq_lens, n_states, out_mode):
-    """The same call in a workspace that ends before the strips' tables."""
-    from tests.gpu_util import DeviceProblem
-    P = DeviceProblem(am, edges, weights, start_end, seq_lens, n_states)
-    P.ws_bytes -= 256
-    out, loss = P.run(out_mode)
-    return out.cpu().numpy(), loss.cpu().numpy()
-
-
 @pytest.mark.parametrize("kind", ["chain", "mixed"])
 def test_a_batch_goes_through_the_strips_as_a_whole(oracle, kind):
     """One sequence that they cannot take, and the others go with it: the two recursions one behind the other would take as
@@ -265,7 +377,7 @@ def test_a_batch_goes_through_the_strips_as_a_whole(oracle, kind):
 
 
 @pytest.mark.parametrize("writer", [0, 1], ids=["rows", "flat"])
-@pytest.mark.parametrize("kind", ["optional", "mixed"])
+@pytest.mark.parametrize("kind", ["passing", "mixed"])
 def test_large_automata_overlapped_or_in_strips(oracle, kind, writer):
     """Calls whose sizes ask for the overlapped schedule: enqueued both ways, the preparation decides."""
     from tests.gpu_util import run_cabi
@@ -274,9 +386,6 @@ def test_large_automata_overlapped_or_in_strips(oracle, kind, writer):
     T, B, F = 1025, 5, 13100
     assert T * B * F >= 1 << 26
     edges, weights, start_end, n = automata(rng, rng.integers(590, 650, size=B).tolist(), F, kind)
-    # (few states can be passed over: 2.3 edges per state is the limit for automata of this size)
-    keep = (edges[1] - edges[0] != 2) | (rng.random(edges.shape[1]) < 0.4)
-    edges, weights = edges[:, keep].copy(), weights[keep].copy()
     am = rng.uniform(0.1, 9.0, size=(T, B, F)).astype(np.float32)
     lens = rng.integers(660, T + 1, size=B).astype(np.int32)
     lens[1] = T
