@@ -19,7 +19,7 @@ N_STAGES = 5
 STAGE_NAMES = ("prepare", "gather", "recurse", "combine", "padfill")
 
 # every symbol include/i6fbw.h declares
-SYMBOLS = ("i6fbw_workspace_size", "i6fbw_run", "i6fbw_run_strided", "i6fbw_read_status", "i6fbw_strerror", "i6fbw_last_hip_error",
+SYMBOLS = ("i6fbw_workspace_size", "i6fbw_workspace_size_for", "i6fbw_run", "i6fbw_run_strided", "i6fbw_read_status", "i6fbw_strerror", "i6fbw_last_hip_error",
            "i6fbw_set_overlap", "i6fbw_viterbi", "i6fbw_dump_output", "i6fbw_dump_alignment",
            "i6fbw_ctc_fsa_bounds", "i6fbw_build_ctc_fsa", "i6fbw_build_hmm_fsa",
            "i6fbw_profile_enable", "i6fbw_profile_read",
@@ -40,6 +40,8 @@ def load():
         c = ctypes
         lib.i6fbw_workspace_size.argtypes = [c.c_int] * 5 + [c.POINTER(c.c_size_t)]
         lib.i6fbw_workspace_size.restype = c.c_int
+        lib.i6fbw_workspace_size_for.argtypes = [c.c_int] * 6 + [c.POINTER(c.c_size_t)]
+        lib.i6fbw_workspace_size_for.restype = c.c_int
         lib.i6fbw_run.argtypes = [c.c_void_p, c.c_int64, c.c_int64, c.c_void_p, c.c_int64, c.c_void_p, c.c_void_p,
                                   c.c_int64, c.c_void_p, c.c_int, c.c_int, c.c_int, c.c_int, c.c_int, c.c_int,
                                   c.c_void_p, c.c_void_p, c.c_void_p, c.c_size_t, c.c_void_p]
@@ -116,6 +118,15 @@ class FbwError(RuntimeError):
 def workspace_size(T, B, F, E, n_states) -> int:
     n = ctypes.c_size_t(0)
     rc = load().i6fbw_workspace_size(T, B, F, E, n_states, ctypes.byref(n))
+    if rc != 0:
+        raise FbwError(rc)
+    return int(n.value)
+
+
+def workspace_size_for(best_path, T, B, F, E, n_states) -> int:
+    """What run (best_path False) or viterbi (True) alone makes use of."""
+    n = ctypes.c_size_t(0)
+    rc = load().i6fbw_workspace_size_for(1 if best_path else 0, T, B, F, E, n_states, ctypes.byref(n))
     if rc != 0:
         raise FbwError(rc)
     return int(n.value)

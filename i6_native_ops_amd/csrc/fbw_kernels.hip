@@ -344,6 +344,31 @@ inline bool best_path_strips(const int B, const int E, const int n_states, const
     return n <= (states > 512 ? 3LL : 1LL) * n_cu;
 }
 
+// Do the sizes of a call ask for the overlapped schedule?  (measured at F = 12001 unless said otherwise, ms per call stage
+// after stage / overlapped)  Full sum: a large dense tensor; a batch whose recursion workgroups leave half of
+// the compute units alone (T=400 B=100 F=5001: 0.33 / 0.36; T=200 B=256 F=5001: 0.34 / 0.43; with
+// up to 64 sequences T=600 B=32: 0.37 / 0.33, T=1000 B=32: 0.62 / 0.52, T=2000 B=16 F=3000: 1.39 /
+// 1.07); not with few frames (there is little recursion to hide: T=200 B=64 0.20 / 0.23, T=300 B=32
+// 0.19 / 0.20) nor, unless the sequences are long, with a handful of sequences (T=1000 B=8: 0.36 /
+// 0.34, T=4000 B=8 with large automata: 3.27 / 2.81).
+inline bool full_sum_overlaps(const int T, const int B, const int F, const int n_cu) {
+    return (long long)T * B * F >= (1LL << 26) && 2 * B <= n_cu / 2 && T >= 384 && (B >= 12 || T >= 1000);
+}
+// Best path: the same, but the search has less to hide -- up to 600 frames, and for a handful of
+// short sequences, the stages in a row measured as fast or up to a third faster.
+inline bool best_path_overlaps(const int T, const int B, const int F, const int n_cu) {
+    return (long long)T * B * F >= (1LL << 26) && 2 * B <= n_cu && T >= 768 && (B >= 12 || T >= 2048);
+}
+// Can a call use the strips' tables of the workspace?  From its sizes, for a whole device (256 compute units).
+inline bool full_sum_wants_strips(const int T, const int B, const int F, const int E, const int n_states) {
+    const int density = F > F_BITMAP_MAX ? 0 : strip_density(T, B, E, 256);
+    if (density == 0 || 100LL * E > (long long)density * n_states) return false;
+    return !full_sum_overlaps(T, B, F, 256) || ((long long)n_states > (long long)BIG_STATES * B && (long long)E > 1100LL * B);
+}
+inline bool best_path_wants_strips(const int T, const int B, const int F, const int E, const int n_states) {
+    return best_path_strips(B, E, n_states, 256, best_path_overlaps(T, B, F, 256));
+}
+
 // Hand-off between kernels that run at the same time (gather -> recursion -> combine).  The
 // L2 caches of the eight XCDs are not coherent with each other inside a kernel, so everything
 // that crosses kernels goes through agent-scope accesses (sc1: written through / read from the
@@ -3792,7 +3817,15 @@ extern "C" {
 
 int i6fbw_workspace_size(int T, int B, int F, int E, int n_states, size_t* bytes) {
     if (!bytes || T <= 0 || B <= 0 || F <= 0 || E < 0 || n_states <= 0) return I6FBW_ERR_INVALID_ARGUMENT;
-    *bytes = make_layout(T, B, E, F).total;
+    const Layout l = make_layout(T, B, E, F);
+    *bytes = full_sum_wants_strips(T, B, F, E, n_states) || best_path_wants_strips(T, B, F, E, n_states) ? l.total : l.base_total;
+    return I6FBW_OK;
+}
+
+int i6fbw_workspace_size_for(int best_path, int T, int B, int F, int E, int n_states, size_t* bytes) {
+    if (!bytes || T <= 0 || B <= 0 || F <= 0 || E < 0 || n_states <= 0) return I6FBW_ERR_INVALID_ARGUMENT;
+    const Layout l = make_layout(T, B, E, F);
+    *bytes = (best_path ? best_path_wants_strips(T, B, F, E, n_states) : full_sum_wants_strips(T, B, F, E, n_states)) ? l.total : l.base_total;
     return I6FBW_OK;
 }
 
@@ -3891,15 +3924,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     const bool big = !dense && (long long)n_states > (long long)BIG_STATES * B;
     // Small problems run stage after stage on the caller's stream; large ones overlap the stages.
     const int forced = static_call ? 0 : g_overlap_mode.load();
-    // By default only where it pays (measured at F = 12001 unless said otherwise, ms per call stage
-    // after stage / overlapped): a large dense tensor; a batch whose recursion workgroups leave half of
-    // the compute units alone (T=400 B=100 F=5001: 0.33 / 0.36; T=200 B=256 F=5001: 0.34 / 0.43; with
-    // up to 64 sequences T=600 B=32: 0.37 / 0.33, T=1000 B=32: 0.62 / 0.52, T=2000 B=16 F=3000: 1.39 /
-    // 1.07); not with few frames (there is little recursion to hide: T=200 B=64 0.20 / 0.23, T=300 B=32
-    // 0.19 / 0.20) nor, unless the sequences are long, with a handful of sequences (T=1000 B=8: 0.36 /
-    // 0.34, T=4000 B=8 with large automata: 3.27 / 2.81).
-    bool overlap = forced >= 0 ? forced != 0
-                               : ((long long)T * B * F >= (1LL << 26) && 2 * B <= P.n_cu / 2 && T >= 384 && (B >= 12 || T >= 1000));
+    bool overlap = forced >= 0 ? forced != 0 : full_sum_overlaps(T, B, F, P.n_cu);
     // The strip kernels take the place of the recursion stage after stage: also where the overlap would pay for the large
     // instance.  (The dump of the forward scores reads rows in the layout of the other kernels.)
     // (strip_density says where they pay; whether all sequences are such automata is found out by the preparation)

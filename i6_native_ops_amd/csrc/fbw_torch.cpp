@@ -71,7 +71,7 @@ static std::vector<torch::Tensor> run(torch::Tensor& am_scores, torch::Tensor& e
     torch::Tensor out = torch::empty(am_scores.sizes(), opts.dtype(torch::kFloat32));      // contiguous, same shape
     torch::Tensor sum_output = torch::empty({T, B}, opts.dtype(torch::kFloat32));
     size_t ws_bytes = 0;
-    int rc = i6fbw_workspace_size(T, B, F, E, (int)num_states, &ws_bytes);
+    int rc = i6fbw_workspace_size_for(0, T, B, F, E, (int)num_states, &ws_bytes);
     TORCH_CHECK(rc == I6FBW_OK, "NativeOp: fbw: ", i6fbw_strerror(rc));
     torch::Tensor workspace = torch::empty({(int64_t)ws_bytes}, opts.dtype(torch::kUInt8));
     hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();

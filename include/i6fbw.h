@@ -56,10 +56,13 @@ enum {
 };
 
 /*
- * Bytes of device workspace i6fbw_run needs for a problem of this size.
+ * Bytes of device workspace for a problem of this size, enough for i6fbw_run and for i6fbw_viterbi.
  * Replaces the three raw cudaMalloc'ed buffers of fbw_op.cu:283-286.
+ * i6fbw_workspace_size_for: what i6fbw_run alone (best_path 0) or i6fbw_viterbi alone (1) makes use of, which can be
+ * a third less: some of the kernels have tables of their own, and not every call can go to them.
  */
 int i6fbw_workspace_size(int T, int B, int F, int E, int n_states, size_t* bytes);
+int i6fbw_workspace_size_for(int best_path, int T, int B, int F, int E, int n_states, size_t* bytes);
 
 /*
  * One FBW loss+posterior evaluation; replaces fbw_cuda (fbw_op.cu:226-393)
@@ -79,7 +82,8 @@ int i6fbw_workspace_size(int T, int B, int F, int E, int n_states, size_t* bytes
  *   out         float [T,B,F] contiguous, written completely         (fbw_op.cu:231,265)
  *   sum_output  float [T,B] contiguous: total -log likelihood of sequence b in every frame
  *               t < seq_lens[b], 0 elsewhere                         (fbw_op.cu:104-135,232)
- *   workspace   device buffer of at least i6fbw_workspace_size bytes, 256-byte aligned
+ *   workspace   device buffer of at least i6fbw_workspace_size (or i6fbw_workspace_size_for(0, ...)) bytes,
+ *               256-byte aligned
  *   stream      hipStream_t to enqueue on (NULL = default stream); the call is asynchronous.
  *               Inside, a large call forks onto library-owned streams (created on first use,
  *               default priority) and joins `stream` again before the call returns, so everything
@@ -132,8 +136,8 @@ int i6fbw_run_strided(const float* am_scores, int64_t am_stride_t, int64_t am_st
  * kernels work in a built-in device buffer of I6FBW_STATIC_WORKSPACE_BYTES that every GPU the
  * library runs on holds until the process ends.  The call allocates nothing (no device or host
  * memory, no streams, no events) and runs all stages one after the other on `stream`.
- * Problems whose workspace (i6fbw_workspace_size) is larger than the built-in buffer are refused
- * with I6FBW_ERR_STATIC_WORKSPACE.  All calls on one GPU share the one buffer: calls that overlap
+ * Problems whose workspace (i6fbw_workspace_size, less the tables that this call does not use) is larger than the
+ * built-in buffer are refused with I6FBW_ERR_STATIC_WORKSPACE.  All calls on one GPU share the one buffer: calls that overlap
  * in time on the same GPU (two streams, two host threads) race; calls on one stream are ordered
  * and safe.  i6fbw_static_workspace hands out the buffer of the current device, e.g. for
  * i6fbw_read_status(buffer, B, stream, ...) after a call.  The first use of either function on a device
@@ -199,7 +203,7 @@ int i6fbw_get_status_mode(void);
  *               the walk back from the end state finds no back-pointer (core.cu:145-177)
  *   scores      float [B]: value of the end state after seq_lens[b] frames, -inf without a path
  *               (core.cu:124-143)
- *   workspace   as for i6fbw_run (i6fbw_workspace_size bytes)
+ *   workspace   as for i6fbw_run (i6fbw_workspace_size bytes, or i6fbw_workspace_size_for(1, ...))
  *
  * Values are computed in the reference's arithmetic, (previous + weight) + score in fp32, and
  * ties go to the edge that comes first in the input, as the reference's compare-and-swap rule

@@ -45,6 +45,24 @@ def test_workspace_size_and_argument_validation():
     assert cabi.load().i6fbw_strerror(-12) != cabi.load().i6fbw_strerror(-13)
 
 
+@pytest.mark.parametrize("T,B,F,E,n,loss,align", [
+    (1000, 32, 12001, 24000, 12032, False, True),      # tied chains, overlapped by its sizes: the full sum has no use for the strips' tables
+    (437, 19, 4499, 6270, 3154, True, True),           # tied chains
+    (1203, 64, 61, 64000, 25792, False, False),        # CTC over characters
+    (300, 128, 264, 46080, 23168, False, True),        # more chains than the strips pay for
+    (200, 32, 264, 11520, 5792, False, True),          # too short
+])
+def test_workspace_holds_the_tables_a_call_can_use(T, B, F, E, n, loss, align):
+    """No more than that: 501 MB, not 719, for the full sum of the first case."""
+    from i6_native_ops_amd import cabi
+    most = cabi.workspace_size(T, B, F, E, n)
+    small = cabi.workspace_size_for(False, T, B, F, E, 1)       # (one state for all those edges: no strips)
+    assert cabi.workspace_size_for(False, T, B, F, E, n) == (most if loss else small)
+    assert cabi.workspace_size_for(True, T, B, F, E, n) == (most if align else small)
+    if T == 1000:
+        assert 490e6 < small < 510e6 and 700e6 < most < 730e6
+
+
 def test_extension_module_surface():
     import i6_native_ops_amd.fbw as fbw
     assert callable(fbw.fbw_loss) and issubclass(fbw.FastBaumWelchLoss, torch.autograd.Function)
