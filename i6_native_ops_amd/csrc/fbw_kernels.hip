@@ -64,6 +64,7 @@ constexpr int TC = I6_TC;             // frames per combine workgroup
 #endif
 constexpr int FLAT_TCF = I6_FLAT_TCF; // frames per posterior job of the flat dense write (one flag each)
 static_assert(TC % FLAT_TCF == 0, "posterior jobs tile a strip");
+static_assert(TC == 8 && TG == 8, "the strip kernels' blocks of eight frames are a gather's and a row writer's strip");
 constexpr int RENORM = 8;             // frames between renormalisations of the state vector
 constexpr int COMB_THREADS = 256;
 constexpr int COMB_JD = D_MAX / COMB_THREADS;
@@ -2359,7 +2360,9 @@ __device__ __forceinline__ bool comb_small(const SeqMeta& m, const int batch) {
 #endif
 constexpr int COMB_SMALL_OCC = I6_COMB_SMALL_OCC;
 // (WIDE: the general instance with the path for more than COMB_XS staged edges in the place of the one in passes)
-template <bool SYNC, bool NEGLOG, bool SMALL = false, bool WIDE = false>
+// (STRIPS: the small instance for calls that may have gone through the strips; in the other one the fold of their offsets, though
+// never taken, cost registers: 256 chains of 375 states 483 -> 493 us)
+template <bool SYNC, bool NEGLOG, bool SMALL = false, bool WIDE = false, bool STRIPS = !SMALL>
 __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_combine(CombArgs a) {
     extern __shared__ float4a lds4[];
     __shared__ float redmin[COMB_THREADS / 64];
@@ -2463,7 +2466,7 @@ __global__ __launch_bounds__(COMB_THREADS, SMALL ? COMB_SMALL_OCC : 3) void fbw_
     const float* bbase = a.beta + (size_t)T * soff;
     const float* gbase = a.gtab + (size_t)T * goff;
     __shared__ StripView view;
-    const bool stripped = !SYNC && strip_view(view, a, m, b, t0 / STRIP_FRAMES);
+    const bool stripped = !SYNC && STRIPS && strip_view(view, a, m, b, t0 / STRIP_FRAMES);
     if (stripped && view.lost) {
         for (int t = t0; t < tv; t++) {
             stream_const_row(a.out + t * a.ost_t + b * a.ost_b, a.F, __builtin_nanf(""));
@@ -3635,17 +3638,23 @@ void launch_prepare(const Pipeline& P, const PrepArgs& pa, hipStream_t s) {
 size_t comb_batch_lds_bytes(int F) { return (size_t)COMB_BATCH * ((size_t)(((F + 32 + 3) >> 2) * 16) + (size_t)COMB_BATCH_EDGES * 4); }
 template <bool SYNC>
 void launch_combine(const bool neglog, const dim3 grid, const size_t lds, hipStream_t s, CombArgs ca) {
+    // (what the general instance stages beyond COMB_XS edges is its alone: with that LDS the small one had two workgroups less
+    // on a unit, 128 automata of 600 states 541 -> 590 us)
+    const size_t general_lds = lds + (ca.xs_cap ? (size_t)(COMB_WIDE_EDGES - COMB_XS + COMB_MID_SLOTS) * 4 : 0);
     if (!ca.direct_only && !ca.tile_w) {
         size_t lds_s = lds;
         if (ca.F <= COMB_BATCH_F) { ca.batch_frames = 1; lds_s = std::max(lds, comb_batch_lds_bytes(ca.F)); }      // (both instances: it decides which takes a sequence)
         CombArgs cs = ca;
-        if (neglog) hipLaunchKernelGGL((fbw_combine<SYNC, true, true>), grid, dim3(COMB_THREADS), lds_s, s, cs);
+        if (!SYNC && ca.strips > 0) {
+            if (neglog) hipLaunchKernelGGL((fbw_combine<false, true, true, false, true>), grid, dim3(COMB_THREADS), lds_s, s, cs);
+            else hipLaunchKernelGGL((fbw_combine<false, false, true, false, true>), grid, dim3(COMB_THREADS), lds_s, s, cs);
+        } else if (neglog) hipLaunchKernelGGL((fbw_combine<SYNC, true, true>), grid, dim3(COMB_THREADS), lds_s, s, cs);
         else hipLaunchKernelGGL((fbw_combine<SYNC, false, true>), grid, dim3(COMB_THREADS), lds_s, s, cs);
         ca.small_elsewhere = 1;
     }
-    if (neglog) hipLaunchKernelGGL((fbw_combine<SYNC, true, false>), grid, dim3(COMB_THREADS), lds, s, ca);
-    else if (!SYNC && ca.xs_cap) hipLaunchKernelGGL((fbw_combine<false, false, false, true>), grid, dim3(COMB_THREADS), lds, s, ca);
-    else hipLaunchKernelGGL((fbw_combine<SYNC, false, false>), grid, dim3(COMB_THREADS), lds, s, ca);
+    if (neglog) hipLaunchKernelGGL((fbw_combine<SYNC, true, false>), grid, dim3(COMB_THREADS), general_lds, s, ca);
+    else if (!SYNC && ca.xs_cap) hipLaunchKernelGGL((fbw_combine<false, false, false, true>), grid, dim3(COMB_THREADS), general_lds, s, ca);
+    else hipLaunchKernelGGL((fbw_combine<SYNC, false, false>), grid, dim3(COMB_THREADS), general_lds, s, ca);
 }
 template <bool SYNC>
 void launch_flat(const bool neglog, const dim3 grid, hipStream_t s, const FlatArgs& fa) {
@@ -3666,7 +3675,8 @@ int device_init(Pipeline& p) {
     for (const void* k : {(const void*)fbw_combine<true, false, false>, (const void*)fbw_combine<false, false, false>,
                           (const void*)fbw_combine<true, true, false>, (const void*)fbw_combine<false, true, false>,
                           (const void*)fbw_combine<true, false, true>, (const void*)fbw_combine<false, false, true>,
-                          (const void*)fbw_combine<true, true, true>, (const void*)fbw_combine<false, true, true>, (const void*)fbw_combine<false, false, false, true>})
+                          (const void*)fbw_combine<true, true, true>, (const void*)fbw_combine<false, true, true>, (const void*)fbw_combine<false, false, false, true>,
+                          (const void*)fbw_combine<false, false, true, false, true>, (const void*)fbw_combine<false, true, true, false, true>})
         HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048));
     hipFuncAttributes attr;
     HIP_TRY(hipFuncGetAttributes(&attr, (const void*)fbw_recurse_dense<true>));
@@ -3990,8 +4000,6 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     ca.out = out; ca.sum_output = sum_output; ca.ost_t = out_stride_t; ca.ost_b = out_stride_b; ca.sync = sync;
     ca.tile_w = tiled ? COMB_TILE_W : 0;
     ca.direct_only = 0;
-    // (the stage-after-stage instance; in the overlapped schedule it is launched for the strips alone, behind the others)
-    const size_t wide_lds = comb_lds + (wide ? (size_t)(COMB_WIDE_EDGES - COMB_XS + COMB_MID_SLOTS) * 4 : 0);
     ca.strips = strips; ca.soffs = (const double*)(ws + l.soffs); ca.sprog = (const int*)(ws + l.sprog);
     // The dense tensor goes out in flat spans (fbw_flat) if it is one contiguous block in either
     // order of frames and sequences, rows are long enough for a span to cut at most two of them,
@@ -4124,9 +4132,9 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
         f.c = c; f.ahead = FLAT_AHEAD_ALONE;
         if (flat) {
             // (the row kernel first: it only has the sequences that are too large for the other one)
-            { StageTimer tm(4, st, timed); launch_combine<false>(neglog, c_grid, wide_lds, st, c); }
+            { StageTimer tm(4, st, timed); launch_combine<false>(neglog, c_grid, comb_lds, st, c); }
             { StageTimer tm(3, st, timed); launch_flat<false>(neglog, flat_grid(f), st, f); }
-        } else { StageTimer tm(3, st, timed); launch_combine<false>(neglog, c_grid, wide_lds, st, c); }
+        } else { StageTimer tm(3, st, timed); launch_combine<false>(neglog, c_grid, comb_lds, st, c); }
         HIP_TRY(hipGetLastError());
         return I6FBW_OK;
     };
