@@ -3558,8 +3558,10 @@ __global__ void fbw_selftest_set(int v) { if (threadIdx.x == 0) store_agent(&g_s
 // Holds back the combine kernel (next on the same stream) until every workgroup of the recursion
 // kernel has been placed on the machine: combine workgroups wait for recursion progress while
 // they occupy LDS and wave slots, so they must not be able to keep a recursion workgroup out.
-__global__ __launch_bounds__(64) void fbw_gate(int* sync, int need) {
-    if (threadIdx.x == 0) spin_until_ge(sync + 1, need, sync);
+// (A batch that the strips take has no work for the kernels behind this one, and nothing to wait for: the recursion's workgroups
+// may find no room before the strips' kernels leave some.)
+__global__ __launch_bounds__(64) void fbw_gate(int* sync, int need, int strips) {
+    if (threadIdx.x == 0 && !strips_on(strips, sync)) spin_until_ge(sync + 1, need, sync);
 }
 
 // Rows of frames t >= seq_len (all rows if seq_len is outside [1, T]): out = hole, sum_output = 0
@@ -3935,9 +3937,9 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // Small problems run stage after stage on the caller's stream; large ones overlap the stages.
     const int forced = static_call ? 0 : g_overlap_mode.load();
     bool overlap = forced >= 0 ? forced != 0 : full_sum_overlaps(T, B, F, P.n_cu);
-    // The strip kernels take the place of the recursion stage after stage: also where the overlap would pay for the large
-    // instance.  (The dump of the forward scores reads rows in the layout of the other kernels.)
-    // (strip_density says where they pay; whether all sequences are such automata is found out by the preparation)
+    // The strip kernels take the place of the recursion stage after stage, and of the overlapped stages where the automata are
+    // large (strip_density says where that pays; whether all sequences are such automata is found out by the preparation).
+    // Not for the dump of the forward scores, which reads rows in the layout of the other kernels.
     const bool strips_large = (long long)E > 1100LL * B;
     const int density = !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strip_density(T, B, E, P.n_cu) : 0;
     int strips = density > 0 && 100LL * E <= (long long)density * n_states ? strips_to_launch(B, strip_states(B, E)) : 0;
@@ -4174,7 +4176,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // held back until every recursion workgroup is on the machine -- normally long since.
     // (Or by the preparation's workgroups at their end, see gate_in_prepare.)
     if (!gate_in_prepare) {
-        hipLaunchKernelGGL(fbw_gate, dim3(1), dim3(64), 0, sG, sync, 2 * B);
+        hipLaunchKernelGGL(fbw_gate, dim3(1), dim3(64), 0, sG, sync, 2 * B, strips);
         HIP_TRY(hipGetLastError());
     }
     { StageTimer tm(1, sG, timed); hipLaunchKernelGGL(fbw_gather<true>, g_grid, dim3(256), 0, sG, ga); }
