@@ -118,6 +118,12 @@ constexpr float LN2 = 0.693147180559945309f;
 constexpr int STRIP_HALO = 4, STRIP_USE = 64 - STRIP_HALO, STRIP_MAX = (S_MAX + STRIP_HALO + STRIP_USE - 1) / STRIP_USE;
 constexpr int STRIP_FRAMES = 8;       // frames per block of the strip kernels
 constexpr int STRIP_DEGREE = 6;       // edges entering or leaving a state that they hold in registers
+// Which score an edge takes, for the strip kernels (SeqMeta::emit, found out by the preparation): that of the state it leaves (HMM chains) or
+// that of the state it enters (CTC), so that a state has one score per frame, or one of its own.  Edges into an end state that no
+// edge leaves are left out of this where they are otherwise (CTC: copies of the edges into the last two states), STRIP_ODD_END:
+// such a state has a value behind the last frame only.  STRIP_MIXED: some other edge raises the state by more than two numbers, or
+// has a twin.
+constexpr int EMIT_MASK = 3, EMIT_EDGE = 0, EMIT_SOURCE = 1, EMIT_TARGET = 2, STRIP_ODD_END = 4, STRIP_MIXED = 8;
 
 struct SeqMeta {
     int edge_begin;   // edges with a smaller sequence index
@@ -131,6 +137,7 @@ struct SeqMeta {
     int Kin, errA;    // written by the target-order role
     int Kout, errB;   // written by the source-order role
     int pad;          // bit 0: edges contiguous in the input; bit 1: states renumbered; bit 2: their numbers stand in a plain array; bits 8 and up: see live_window
+    int emit;         // where the strip kernels take the batch, see EMIT_MASK
 };
 
 __host__ __device__ inline long long round16(long long x) { return (x + 15) & ~15LL; }
@@ -149,7 +156,7 @@ __host__ __device__ inline unsigned renum_home(int id, unsigned cap) {
 }
 
 struct Layout {
-    size_t meta, sync, sortflag, seqbegin, eidx, ellA, ellB, crec, cbegin, demis, tband, renum, cflag, wpfx, offA, offB, alpha, beta, gtab, base_total, sprog, soffs, shalo, etab, total;
+    size_t meta, sync, sortflag, seqbegin, eidx, ellA, ellB, crec, cbegin, demis, tband, renum, cflag, wpfx, offA, offB, alpha, beta, gtab, base_total, sprog, soffs, shalo, sslot, etab, total;
     long long ss_total, gg_total;
     int wpfx_stride;      // ints per sequence in the emission rank table (0: F too large for it)
 };
@@ -187,6 +194,7 @@ Layout make_layout(long long T, long long B, long long E, long long F = 1) {
     l.sprog = o;    o = align256(o + sizeof(int) * 2 * STRIP_MAX * B);
     l.soffs = o;    o = align256(o + sizeof(double) * 2 * STRIP_MAX * B * ((T + 7) / 8));
     l.shalo = o;    o = align256(o + sizeof(double) * 2 * STRIP_HALO * (strip_border_off(E, (int)B) + 2) * (((size_t)T + 7) & ~(size_t)7));
+    l.sslot = o;    o = align256(o + sizeof(unsigned short) * l.ss_total);
     l.etab = o;     o = align256(o + sizeof(float) * (strip_off(E, (int)B) + 16) * (((size_t)T + 7) & ~(size_t)7));
     l.total = o;
     return l;
@@ -232,6 +240,13 @@ __device__ inline int rec_class(const SeqMeta& m, const int threads = REC_THREAD
 
 // Number of strips of S states
 __host__ __device__ inline int strips_of(const int S) { return (S + STRIP_HALO + STRIP_USE - 1) / STRIP_USE; }
+// Best path over strips, a sequence's share of alpha's area: back-pointers (64 bytes per strip and frame), halo values (16), and per
+// chunk of CHUNK_BLOCKS blocks where a path that is in a state behind the chunk was in front of it (two bytes) and, from a new cache line on, the
+// state of the best one
+constexpr int CHUNK_BLOCKS = 8, CHUNK_FRAMES = CHUNK_BLOCKS * STRIP_FRAMES;
+__host__ __device__ inline long long vit_strip_bytes(const long long n, const long long T8, const long long T, const long long SP) {
+    return 80 * n * T8 + (T + CHUNK_FRAMES - 1) / CHUNK_FRAMES * (2 * SP + 4) + 128;
+}
 // Can the strip kernels (strip_kernels.inc) take an automaton?  They need states numbered so that no edge leads downward (d: by
 // how much one raises the number at most, 0 where that is not so) and none raises the number by more than the halo, and
 // tables that fit the sequence's share of the workspace; `most` is what the host has launched waves for.
@@ -240,9 +255,14 @@ __device__ inline bool strip_shape(const int S, const int n_edges, const int edg
     if (d < 1 || d > STRIP_HALO || n > most) return false;
     if (64LL * (d == 1 ? 2 : 3) * n > strip_off(edge_begin + n_edges, b + 1) - strip_off(edge_begin, b)) return false;
     if ((n - 1) / 4 > strip_border_off(edge_begin + n_edges, b + 1) - strip_border_off(edge_begin, b)) return false;
-    // (alpha's area also holds back-pointers and halo values of the best-path search: 80 bytes per strip and frame)
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
-    return 80LL * n * T8 <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
+    return vit_strip_bytes(n, T8, T, round16(S)) <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
+}
+// The rows of the best path (64 floats per strip and frame) stand behind the score of a state in the strips' score table, or in beta's area
+// where every edge has a score of its own.
+__device__ inline bool vit_rows_fit(const int S, const int n_edges, const int edge_begin, const int b, const int T, const int emit) {
+    const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
+    return emit != EMIT_EDGE || 64LL * strips_of(S) * T8 <= T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
 }
 // A batch goes through the strips as a whole or not at all: with some of its sequences left to the other recursion (or search),
 // which then runs behind the strips, a call took as long as both (8 sequences of 510-690 states, some of them on the other
@@ -468,7 +488,9 @@ struct PrepArgs {
     int strips = 0;         // > 0: a batch of sequences of up to that many strips goes to the strip kernels ...
     int strip_density = 0;  // ... if none has more than this many edges per 100 states (0: any number)
     int level = 0;          // 1: every sequence whose ids do not follow the automaton gets numbers along it; 2: those of at most strip_density edges per 100 states
+    unsigned short* sslot = nullptr;   // per state: slot of its score, where it has one (STRIP_EMIT)
     int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence; the last one is the mark of strip_lost
+    int roles() const { return strips > 0 && !best_path ? 4 : 3; }      // workgroups per sequence
 };
 
 // sortflag[blk] = 1 if the sequence indices of edges [blk*SCAN_BLOCK, (blk+1)*SCAN_BLOCK] never
@@ -614,7 +636,7 @@ __device__ inline int min_steps(int from, int to, int dmax, int dmin) {
     return dmin < 0 ? (-diff - dmin - 1) / -dmin : (1 << 30);
 }
 
-// grid (3, B): role 0 orders the edges of sequence b by target state (alpha), role 1 by source
+// grid (3 or 4, B): role 0 orders the edges of sequence b by target state (alpha), role 1 by source
 // state (beta), role 2 by emission slot (combine) and writes the shared part of the meta record.
 // For edge lists grouped by sequence (the usual case) the scan kernel has recorded where each
 // sequence starts; any other order is handled by a stable scan over the whole list.
@@ -988,15 +1010,80 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         return;
     }
 
-    if (a.best_path && role == 1) {
-        if (tid == 0) { a.meta[b].Kout = 0; a.meta[b].errB = 0; }
-        return;
-    }
+    if (a.best_path && role == 1 && tid == 0) { a.meta[b].Kout = 0; a.meta[b].errB = 0; }
     const float wscale = a.best_path ? 1.f : LOG2E;
 
     auto slot_of = [&](unsigned em) -> unsigned {
         return (unsigned)wordpfx[em >> 5] + (unsigned)__popc(bitmap[em >> 5] & ((1u << (em & 31)) - 1u));
     };
+
+    if (role == (a.best_path ? 1 : 3)) {
+        if (a.strips == 0) return;
+        // What the strip kernels want to know about the edges (EMIT_MASK), and the states' slots.  A role of its own: 3 us behind the others' work.
+        // Lower half of the sort keys: a slot of the edges that leave a state; of those that enter it, with a bit for every number
+        // that one of them raises the state by.
+        unsigned short* src = (unsigned short*)keys;
+        unsigned short* tgt = src + S_MAX;
+        constexpr unsigned NO_SLOT = 0xFFFFu, SLOT = 0xFFFu;
+        static_assert(S_MAX <= EB_MAX / 2 && D_MAX <= SLOT + 1, "two arrays of 16 bits; twelve bits of slot, three of numbers");
+        enum { SRC = 1, TGT = 2, MIXED = 4, END_SRC = 8, END_TGT = 16, END_MIXED = 32, STEEP = 64 };
+        constexpr int EPT = EB_MAX / NT;
+        unsigned ends[EPT];                  // source | target << 16
+        unsigned short slots[EPT];
+        int found = 0, leaves = 0;
+        for (int s = tid; s < (int)S; s += NT) { src[s] = (unsigned short)NO_SLOT; tgt[s] = 0; }
+#pragma unroll
+        for (int j = 0; j < EPT; j++) {
+            if (j * NT >= n_edges) break;
+            if (tid + j * NT < n_edges) {
+                const int e = edge_at(tid + j * NT), u = (int)local((unsigned)e_from[e]), v = (int)local((unsigned)e_to[e]);
+                ends[j] = (unsigned)u | ((unsigned)v << 16);
+                slots[j] = (unsigned short)slot_of((unsigned)e_emis[e]);
+                leaves |= u == end_loc;
+                if (v < u || v - u > STRIP_HALO) found |= STEEP;
+            }
+        }
+        if (tid == 0) s_count = 0;
+        const bool terminal = !__syncthreads_or(leaves);
+        // any slot of a state, then whether all its edges have that one; the edges into a terminal end state behind the others
+#pragma unroll
+        for (int pass = 0; pass < 2; pass++) {
+            auto mine = [&](const int j) { return tid + j * NT < n_edges && (terminal && (int)(ends[j] >> 16) == end_loc) == (pass == 1); };
+#pragma unroll
+            for (int j = 0; j < EPT; j++) {
+                if (j * NT >= n_edges) break;
+                if (!mine(j)) continue;
+                const int u = (int)(ends[j] & 0xFFFFu), v = (int)(ends[j] >> 16);
+                if (pass == 0 || src[u] == NO_SLOT) src[u] = slots[j];
+                tgt[v] = slots[j];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < EPT; j++) {
+                if (j * NT >= n_edges) break;
+                if (!mine(j)) continue;
+                const int u = (int)(ends[j] & 0xFFFFu), v = (int)(ends[j] >> 16), at = 12 + 16 * (v & 1);
+                if (src[u] != slots[j]) found |= pass ? END_SRC : SRC;
+                if ((tgt[v] & SLOT) != slots[j]) found |= pass ? END_TGT : TGT;
+                const int raise = v - u;
+                if (raise < 0 || raise > 2 || ((atomicOr((unsigned*)(tgt + (v & ~1)), 1u << (at + raise)) >> (at + raise)) & 1u)) found |= pass ? END_MIXED : MIXED;
+            }
+        }
+        if (found) atomicOr(&s_count, found);
+        __syncthreads();
+        found = s_count;
+        const bool by_source = !(found & SRC), by_target = !(found & TGT);
+        const int emit = by_source && (!by_target || !(found & END_SRC)) ? EMIT_SOURCE : by_target ? EMIT_TARGET : EMIT_EDGE;
+        const bool odd_end = (found & END_MIXED) || (emit == EMIT_SOURCE && (found & END_SRC)) || (emit == EMIT_TARGET && (found & END_TGT));
+        if (tid == 0) a.meta[b].emit = emit | (odd_end ? STRIP_ODD_END : 0) | ((found & MIXED) ? STRIP_MIXED : 0);
+        if ((found & STEEP) || (a.best_path && !vit_rows_fit((int)S, n_edges, edge_begin, b, a.T, emit))) uncovered();
+        unsigned short* ss = a.sslot + soff;
+        for (int s = tid; s < SP; s += NT) {
+            const unsigned x = s >= (int)S ? 0u : emit == EMIT_SOURCE ? src[s] : tgt[s] & SLOT;
+            ss[s] = (unsigned short)(x == NO_SLOT ? 0u : x);
+        }
+        return;
+    }
 
     // sort keys: (primary << 13) | position in input order; ties keep the input order
     int N = NT;                       // at least one key per thread, see below
@@ -3629,8 +3716,8 @@ void launch_prepare(const Pipeline& P, const PrepArgs& pa, hipStream_t s) {
     // 512 threads: four workgroups per compute unit for large batches (one round instead of two), and for sequences of up
     // to 512 edges on average, which have no work for more (fewer waves at every barrier: 50 x 2 x 10 0.058 -> 0.052 ms per
     // call, 500 x 32 x 264 0.178 -> 0.173; 750 edges per sequence: no difference; 256 threads: slower from 380 edges on)
-    if (3 * pa.B > 2 * P.n_cu || (long long)pa.E <= 512LL * pa.B) hipLaunchKernelGGL(fbw_prepare<512>, dim3(3, pa.B), dim3(512), lds, s, pa);
-    else hipLaunchKernelGGL(fbw_prepare<1024>, dim3(3, pa.B), dim3(1024), lds, s, pa);
+    if (3 * pa.B > 2 * P.n_cu || (long long)pa.E <= 512LL * pa.B) hipLaunchKernelGGL(fbw_prepare<512>, dim3(pa.roles(), pa.B), dim3(512), lds, s, pa);
+    else hipLaunchKernelGGL(fbw_prepare<1024>, dim3(pa.roles(), pa.B), dim3(1024), lds, s, pa);
 }
 
 // The dense writers, in the instance for the output mode (NEGLOG: the -log output, summed in log space)
@@ -3979,7 +4066,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     pa.ellA = (uint2*)(ws + l.ellA); pa.ellB = (uint2*)(ws + l.ellB);
     pa.crec = (uint4*)(ws + l.crec); pa.cbegin = (int*)(ws + l.cbegin); pa.demis = (int*)(ws + l.demis); pa.tband = (int2*)(ws + l.tband);
     pa.cflag = (int*)(ws + l.cflag); pa.wpfx = l.wpfx_stride > 0 ? (int*)(ws + l.wpfx) : nullptr; pa.wpfx_stride = l.wpfx_stride;
-    pa.strips = strips; pa.strip_density = density; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog);
+    pa.strips = strips; pa.strip_density = density; pa.level = strips > 0 && strips_large ? 2 : 0; pa.sprog = (int*)(ws + l.sprog); pa.sslot = (unsigned short*)(ws + l.sslot);
     GatherArgs ga;
     ga.am = am; ga.st_t = am_stride_t; ga.st_b = am_stride_b; ga.T = T; ga.B = B;
     ga.meta = meta; ga.demis = pa.demis; ga.tband = pa.tband; ga.gtab = (float*)(ws + l.gtab); ga.sync = sync;
@@ -3990,7 +4077,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     gen.all_frames = (input_flags & I6FBW_IN_ALL_FRAMES) ? 1 : 0;
     RecArgs ra;
     ra.gen = gen;
-    ra.T = T; ra.B = B; ra.prep_wgs = 3 * B; ra.meta = meta; ra.ellA = pa.ellA; ra.ellB = pa.ellB; ra.gtab = ga.gtab; ra.gtab_rw = ga.gtab;
+    ra.T = T; ra.B = B; ra.prep_wgs = pa.roles() * B; ra.meta = meta; ra.ellA = pa.ellA; ra.ellB = pa.ellB; ra.gtab = ga.gtab; ra.gtab_rw = ga.gtab;
     ra.alpha = (float*)(ws + l.alpha); ra.beta = (float*)(ws + l.beta);
     ra.strips = strips;
     ra.offA = (double*)(ws + l.offA); ra.offB = (double*)(ws + l.offB); ra.sync = sync;
@@ -4117,7 +4204,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // Gather and recursion over strips, for batches that can be cut that way (the kernels find that out by themselves).
     auto launch_strips = [&](hipStream_t st) -> int {
         StripGatherArgs sg;
-        sg.g = ga; sg.ell = pa.ellA; sg.etab = (float*)(ws + l.etab); sg.strips = strips; sg.cap = strip_gather_lds(B, E); sg.keep_rows = 1; sg.soffs = (double*)(ws + l.soffs);
+        sg.g = ga; sg.ell = pa.ellA; sg.etab = (float*)(ws + l.etab); sg.sslot = pa.sslot; sg.strips = strips; sg.cap = strip_gather_lds(B, E); sg.keep_rows = 1; sg.soffs = (double*)(ws + l.soffs);
         sg.strips_only = overlap ? 1 : 0;
         FbwStripArgs sa;
         sa.T = T; sa.B = B; sa.strips = strips; sa.meta = meta; sa.ellA = pa.ellA; sa.ellB = pa.ellB; sa.gtab = ga.gtab; sa.etab = sg.etab;
