@@ -346,8 +346,16 @@ inline long long strip_groups(const long long states) { return (strips_of((int)s
 //   560 states 0.89 at n=192, 1.09 at 384; 900 0.86 at 256, 0.98 at 512; 1300-1750 0.84 at 384-512, 1.05 at 768-1024
 //   2.6 edges per state: as with 2.14 -- the line is at 2.3 because CTC automata have 2.5 less their repeated labels: with the
 //   edges into their last state a wave takes 540 ns a frame (301 states 1.27-1.34, 601 states 0.99-1.24)
-inline int strip_density(const int T, const int B, const int E, const int n_cu) {
+inline int strip_density(const int T, const int B, const int E, const int n_states, const int n_cu) {
     if (T < 256) return 0;
+    if (250LL * n_states < 100LL * E && 100LL * E <= 310LL * n_states) {
+        // CTC automata at the capacity of their builder (three edges per state on the host's side, 2.5 less repeated labels on the device's).  Call with strips /
+        // without (a workgroup per sequence, three to six candidates per state; what the strips cost is 190 ns a frame): 64 sequences of 200-600 states, T=1203: 810 / 942
+        // us (recursion 540 -> 250); 1 of 400 and 630, T=2302 and 3576: 486 / 1162, 699 / 1950; 10 of 1200, T=3746: 1661 / 3103; 59 of 260, T=516: 251 / 315; 16 of
+        // 80, T=300 F=50000: 289 / 311.
+        const long long states = std::min(strip_states(B, E), (long long)n_states / B + 1), n = 2LL * B * strip_groups(states);
+        return n <= (states > 256 ? 3 * n_cu / 2 : n_cu / 2) ? 310 : 0;
+    }
     const long long states = strip_states(B, E), n = 2LL * B * strip_groups(states);
     if ((long long)E > 1100LL * B && n <= (states > 1024 ? 2LL : 1LL) * n_cu) return 230;
     const long long most = states < 96 ? 0 : states <= 480 ? (states > 256 ? n_cu : T >= 384 ? n_cu / 2 : n_cu / 4) : (states > 720 ? 4LL : 2LL) * n_cu;
@@ -382,7 +390,7 @@ inline bool best_path_overlaps(const int T, const int B, const int F, const int 
 }
 // Can a call use the strips' tables of the workspace?  From its sizes, for a whole device (256 compute units).
 inline bool full_sum_wants_strips(const int T, const int B, const int F, const int E, const int n_states) {
-    const int density = F > F_BITMAP_MAX ? 0 : strip_density(T, B, E, 256);
+    const int density = F > F_BITMAP_MAX ? 0 : strip_density(T, B, E, n_states, 256);
     if (density == 0 || 100LL * E > (long long)density * n_states) return false;
     return !full_sum_overlaps(T, B, F, 256) || ((long long)n_states > (long long)BIG_STATES * B && (long long)E > 1100LL * B);
 }
@@ -4028,7 +4036,7 @@ int run_impl(const float* am, int64_t am_stride_t, int64_t am_stride_b, int inpu
     // large (strip_density says where that pays; whether all sequences are such automata is found out by the preparation).
     // Not for the dump of the forward scores, which reads rows in the layout of the other kernels.
     const bool strips_large = (long long)E > 1100LL * B;
-    const int density = !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strip_density(T, B, E, P.n_cu) : 0;
+    const int density = !static_call && workspace_bytes >= l.total && !f_too_large && !(input_flags & I6FBW_IN_ALL_FRAMES) ? strip_density(T, B, E, n_states, P.n_cu) : 0;
     int strips = density > 0 && 100LL * E <= (long long)density * n_states ? strips_to_launch(B, strip_states(B, E)) : 0;
     // All 2B recursion workgroups must be on the machine at the same time (at most two per compute
     // unit): gather and dense write wait for their progress while occupying wave slots themselves.

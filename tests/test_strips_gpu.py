@@ -194,6 +194,41 @@ def test_full_sum(oracle, case, permute):
     check_full_sum(oracle, args, strips=not (permute and case in (0, 1, 4)))
 
 
+@pytest.mark.parametrize("n_frames", [257, 258, 263, 264])
+def test_full_sum_last_state_alone_in_a_strip(oracle, n_frames):
+    """Backward strips hold the states from 60 j - 4 on: with 57 states more than a multiple of 60 the end state has the last one to
+    itself, and a value in a single row."""
+    rng = np.random.default_rng(500 + n_frames)
+    edges, weights, start_end, n = automata(rng, [117, 177, 237], 40, "chain")
+    am = rng.uniform(0.1, 9.0, size=(264, 3, 40)).astype(np.float32)
+    check_full_sum(oracle, (am, edges, -weights, start_end, np.array([n_frames, 264, n_frames], dtype=np.int32), n))
+
+
+@pytest.mark.parametrize("labels", [(27, 30, 28, 29), (57, 58, 87, 60), (119, 147, 118, 120), (260, 300, 297, 290)])
+def test_full_sum_ctc(oracle, labels):
+    """CTC automata as ctc_fsa leaves them (arrays at their capacity): an end state with five entering edges, alone in a strip or beside others, and
+    last frames everywhere in a block; a repeated label at the end."""
+    from i6_native_ops_amd.fsa import ctc_fsa
+    from tests.gpu_util import DeviceProblem
+    from tests.helpers import posterior
+    rng = np.random.default_rng(sum(labels))
+    F, T = 23, max(272, 5 * max(labels) // 2)
+    lens = np.array([T, T - 3, T - 8, T - 9], dtype=np.int32)
+    targets = rng.integers(1, F, size=(4, max(labels))).astype(np.int32)
+    targets[2, labels[2] - 2] = targets[2, labels[2] - 1]
+    am = rng.uniform(0.1, 9.0, size=(T, 4, F)).astype(np.float32)
+    n, edges, weights, start_end = (x.cpu().numpy() if torch.is_tensor(x) else x for x in
+                                    ctc_fsa(torch.from_numpy(targets).cuda(), torch.from_numpy(np.array(labels, dtype=np.int32)).cuda()))
+    there = edges[3] >= 0
+    want_out, want_loss = oracle.fbw_oracle(am, edges[:, there].copy(), weights[there].copy(), start_end, lens, int(n), threads=4)
+    P = DeviceProblem(am, edges, weights, start_end, lens, n)
+    strips = P.run(cabi.OUT_PROB)[0].cpu().numpy()
+    np.testing.assert_allclose(P.loss.cpu().numpy(), want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(strips, posterior(want_out), rtol=0, atol=1e-4)
+    P.ws_bytes -= 256       # without the strips' tables: other bits show that they were there
+    assert not np.array_equal(strips, P.run(cabi.OUT_PROB)[0].cpu().numpy())
+
+
 def test_full_sum_over_impossible_scores(oracle):
     """Scores of +inf (probability 0): scattered ones, a class that is never possible, a frame that lets nothing pass."""
     rng = np.random.default_rng(31)
