@@ -255,6 +255,7 @@ __device__ inline bool strip_shape(const int S, const int n_edges, const int edg
     if (d < 1 || d > STRIP_HALO || n > most) return false;
     if (64LL * (d == 1 ? 2 : 3) * n > strip_off(edge_begin + n_edges, b + 1) - strip_off(edge_begin, b)) return false;
     if ((n - 1) / 4 > strip_border_off(edge_begin + n_edges, b + 1) - strip_border_off(edge_begin, b)) return false;
+    if (4LL * T * round16(S) >= 1LL << 31) return false;       // (rows through a buffer descriptor, FbwRows)
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
     return vit_strip_bytes(n, T8, T, round16(S)) <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
 }
