@@ -343,10 +343,9 @@ inline long long strip_groups(const long long states) { return (strips_of((int)s
 //                                 1.03 from 128 on; over 500-1000 frames 180-240 states 0.80-0.95 up to 128, 1.07 at 192
 //   375 states, T=1000:           0.74 ... 0.94 at n=256, 1.12 at 384
 //   500 and 560 states, T=1000:   0.57 ... 0.85 and 0.97 at n=576, 0.92 and 1.01 at 768;  900-1750 states: 0.42 ... 0.83 at 1024
-//   2.14 edges per state, 375 states: 0.79 ... 1.05 at n=256, but 180 states 1.02 at n=64 (strip_gather writes three scores per state);
+//   2.14 edges per state, 375 states: 0.79 ... 1.05 at n=256, but 180 states 1.02 at n=64 (with a score per class of edge; one per state: 2 % less);
 //   560 states 0.89 at n=192, 1.09 at 384; 900 0.86 at 256, 0.98 at 512; 1300-1750 0.84 at 384-512, 1.05 at 768-1024
-//   2.6 edges per state: as with 2.14 -- the line is at 2.3 because CTC automata have 2.5 less their repeated labels: with the
-//   edges into their last state a wave takes 540 ns a frame (301 states 1.27-1.34, 601 states 0.99-1.24)
+//   2.6 edges per state: as with 2.14; CTC below
 inline int strip_density(const int T, const int B, const int E, const int n_states, const int n_cu) {
     if (T < 256) return 0;
     if (250LL * n_states < 100LL * E && 100LL * E <= 310LL * n_states) {
@@ -364,7 +363,7 @@ inline int strip_density(const int T, const int B, const int E, const int n_stat
 }
 // Best path: the same question.  Call with strips / without: chains and 2.14 edges per state, 60-180 states 0.62 ... 0.95 and 0.99 at n=256;
 // 375 states 0.60 ... 0.86 at n=256, 0.99 at 384, 1.11 at 512; 900 states 0.43 ... 0.70 at 768; 1750 states 0.27 ... 0.87 at 768, 1.16
-// at 1024.  More than 2.4 edges per state (CTC, whose last strip has edges of any kind, or all strips of that kind): 81 states
+// at 1024.  More than 2.4 edges per state (measured with edges of any kind in CTC's last strip, which it no longer has): 81 states
 // 0.95 up to n=64, 1.02 at 96, 1.07 at 128; 201 and 401 states 0.77 ... 0.86-0.99 at 64, 1.02-1.05 at 128; 551-851 states 0.50 ... 0.80 at 256,
 // 1.02 at 384; 1001 states 0.46 ... 0.53 at 1280 (more than 1024 states of that degree: 3.4 us a frame in the search);
 // five edges per state, 375 states: 0.95 up to 32, 1.01 at 64, 1.5 beyond 256; and slower than the search beside the gather (1.09).
@@ -1085,7 +1084,8 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         const int emit = by_source && (!by_target || !(found & END_SRC)) ? EMIT_SOURCE : by_target ? EMIT_TARGET : EMIT_EDGE;
         const bool odd_end = (found & END_MIXED) || (emit == EMIT_SOURCE && (found & END_SRC)) || (emit == EMIT_TARGET && (found & END_TGT));
         if (tid == 0) a.meta[b].emit = emit | (odd_end ? STRIP_ODD_END : 0) | ((found & MIXED) ? STRIP_MIXED : 0);
-        if ((found & STEEP) || (a.best_path && !vit_rows_fit((int)S, n_edges, edge_begin, b, a.T, emit))) uncovered();
+        // (edges of any kind take 540 ns a frame: more than the other recursion where the automata have as many edges as CTC's)
+        if ((found & STEEP) || (a.strip_density > 230 && (found & MIXED)) || (a.best_path && !vit_rows_fit((int)S, n_edges, edge_begin, b, a.T, emit))) uncovered();
         unsigned short* ss = a.sslot + soff;
         for (int s = tid; s < SP; s += NT) {
             const unsigned x = s >= (int)S ? 0u : emit == EMIT_SOURCE ? src[s] : tgt[s] & SLOT;
