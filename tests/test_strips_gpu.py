@@ -96,6 +96,32 @@ def test_best_path(oracle, case, permute):
     assert_identical((align, scores), oracle.viterbi_oracle(*args))
 
 
+@pytest.mark.parametrize("B", [1, 8])
+@pytest.mark.parametrize("n_frames", [9, 16, 23, 50, 64, 127, 200, 249, 256])
+def test_best_path_of_short_ctc_automata(oracle, n_frames, B):
+    """Up to 256 frames one workgroup follows the path as a whole, from an end state whose edges are looked up apart from the others': last frames
+    everywhere in a block, short sequences behind long ones, repeated labels at the end, scores with and without ties."""
+    from i6_native_ops_amd.fsa import ctc_fsa
+    rng = np.random.default_rng(10 * n_frames + B)
+    F = 29
+    for rep in range(4):
+        # (one sequence: another residue on every turn; eight of them: all residues at once)
+        lens = np.array([max(1, n_frames - (b + 2 * rep) % 8) if b < 6 or rep % 2 else n_frames // 4 + b // 2 for b in range(B)], dtype=np.int32)
+        n_labels = np.array([rng.integers(1, max(2, n // 2)) for n in lens], dtype=np.int32)
+        targets = rng.integers(1, F, size=(B, int(n_labels.max()))).astype(np.int32)
+        for b in range(0, B, 3):
+            if n_labels[b] > 1:
+                targets[b, n_labels[b] - 2] = targets[b, n_labels[b] - 1]
+        am = rng.normal(size=(n_frames, B, F)).astype(np.float32)
+        if rep >= 2:
+            am = np.round(2 * am) / 4
+        n, edges, weights, start_end = (x.cpu().numpy() if torch.is_tensor(x) else x for x in
+                                        ctc_fsa(torch.from_numpy(targets).cuda(), torch.from_numpy(n_labels).cuda()))
+        there = edges[3] >= 0
+        got = run_cabi_viterbi(am, edges, weights, start_end, lens, int(n))
+        assert_identical(got[:2], oracle.viterbi_oracle(am, edges[:, there].copy(), weights[there].copy(), start_end, lens, int(n)))
+
+
 def test_scores_that_are_not_numbers():
     """A NaN never wins, -inf closes an edge, a class of +inf takes everything: as in the other kernels (the reference's
     compare-and-swap does something else with a NaN)."""
