@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "../../include/i6fbw.h"
+#include "strip_rows.h"
 
 namespace {
 
@@ -116,7 +117,6 @@ constexpr float LN2 = 0.693147180559945309f;
 // Strips of states (strip_kernels.inc): lanes of a wave that repeat the last states of the strip before (the first ones of
 // the strip behind, walking backward), states a strip advances by, largest number of strips of one sequence
 constexpr int STRIP_HALO = 4, STRIP_USE = 64 - STRIP_HALO, STRIP_MAX = (S_MAX + STRIP_HALO + STRIP_USE - 1) / STRIP_USE;
-constexpr int STRIP_FRAMES = 8;       // frames per block of the strip kernels
 constexpr int STRIP_DEGREE = 6;       // edges entering or leaving a state that they hold in registers
 // Which score an edge takes, for the strip kernels (SeqMeta::emit, found out by the preparation): that of the state it leaves (HMM chains) or
 // that of the state it enters (CTC), so that a state has one score per frame, or one of its own.  Edges into an end state that no
@@ -255,7 +255,7 @@ __device__ inline bool strip_shape(const int S, const int n_edges, const int edg
     if (d < 1 || d > STRIP_HALO || n > most) return false;
     if (64LL * (d == 1 ? 2 : 3) * n > strip_off(edge_begin + n_edges, b + 1) - strip_off(edge_begin, b)) return false;
     if ((n - 1) / 4 > strip_border_off(edge_begin + n_edges, b + 1) - strip_border_off(edge_begin, b)) return false;
-    if (4LL * T * round16(S) >= 1LL << 31) return false;       // (rows through a buffer descriptor, FbwRows)
+    if (!strip_rows_fit(T, round16(S))) return false;
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
     return vit_strip_bytes(n, T8, T, round16(S)) <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
 }
