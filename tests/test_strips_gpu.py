@@ -96,6 +96,18 @@ def test_best_path(oracle, case, permute):
     assert_identical((align, scores), oracle.viterbi_oracle(*args))
 
 
+def test_best_path_over_many_chunks(oracle):
+    """Where the paths lead over a chunk of 64 frames is written by one workgroup and read by another, in the same kernel and, for most numbers of states,
+    from cache lines that several have written: other scores in the same workspace, again and again."""
+    rng = np.random.default_rng(41)
+    sizes = [30, 70, 100, 130, 175, 250, 330, 10]
+    edges, weights, start_end, n = automata(rng, sizes, 50, "optional")
+    for rep in range(6):
+        am = rng.normal(size=(1500, len(sizes), 50)).astype(np.float32)
+        args = (am, edges, weights, start_end, rng.integers(1300, 1501, size=len(sizes)).astype(np.int32), n)
+        assert_identical(run_cabi_viterbi(*args)[:2], oracle.viterbi_oracle(*args))
+
+
 @pytest.mark.parametrize("B", [1, 8])
 @pytest.mark.parametrize("n_frames", [9, 16, 23, 50, 64, 127, 200, 249, 256])
 def test_best_path_of_short_ctc_automata(oracle, n_frames, B):
