@@ -250,12 +250,12 @@ __host__ __device__ inline long long vit_strip_bytes(const long long n, const lo
 // Can the strip kernels (strip_kernels.inc) take an automaton?  They need states numbered so that no edge leads downward (d: by
 // how much one raises the number at most, 0 where that is not so) and none raises the number by more than the halo, and
 // tables that fit the sequence's share of the workspace; `most` is what the host has launched waves for.
-__device__ inline bool strip_shape(const int S, const int n_edges, const int edge_begin, const int b, const int T, const int d, const int most) {
+__device__ inline bool strip_shape(const int S, const int n_edges, const int edge_begin, const int b, const int T, const int d, const int most, const bool best_path) {
     const int n = strips_of(S);
     if (d < 1 || d > STRIP_HALO || n > most) return false;
     if (64LL * (d == 1 ? 2 : 3) * n > strip_off(edge_begin + n_edges, b + 1) - strip_off(edge_begin, b)) return false;
     if ((n - 1) / 4 > strip_border_off(edge_begin + n_edges, b + 1) - strip_border_off(edge_begin, b)) return false;
-    if (!strip_rows_fit(T, round16(S))) return false;
+    if (!strip_rows_taken(best_path, T, round16(S))) return false;
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
     return vit_strip_bytes(n, T8, T, round16(S)) <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
 }
@@ -1217,7 +1217,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
         if (tid == 0 && d > 0) a.meta[b].pad |= d << 8;
         // (the states counted here: n_states, which the host has, can be any number of times as large where ids are spread, and the
         // same automaton is to take the same kernels, and give the same bits, whatever its ids)
-        if (!strip_shape((int)S, n_edges, edge_begin, b, a.T, d, a.strips) || (a.strip_density > 0 && 100LL * n_edges > (long long)a.strip_density * S)) uncovered();
+        if (!strip_shape((int)S, n_edges, edge_begin, b, a.T, d, a.strips, a.best_path) || (a.strip_density > 0 && 100LL * n_edges > (long long)a.strip_density * S)) uncovered();
         // one thread per edge; the per-slot minimum / maximum is taken with LDS atomics in the
         // memory of the sort keys (and of the distinct ids of a renumbered sequence), which is not
         // needed any more once each thread has worked out the frames of its own edges

@@ -15,3 +15,5 @@ constexpr unsigned STRIP_NO_COLUMN = 0x80000000u;
 I6_ROW_FN unsigned strip_row_offset(const unsigned column, const int t, const int SP) { return column + (unsigned)t * (unsigned)SP * 4u; }
 // Can the offsets of whole blocks of rows be told apart?  All rows together end below STRIP_NO_COLUMN, so that no row takes it around to the first ones.
 I6_ROW_FN bool strip_rows_fit(const long long T, const long long SP) { return 4LL * ((T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES) * SP < (long long)STRIP_NO_COLUMN; }
+// Do the strips take an automaton with that many rows?  The best path stores none of them (its tables are addressed in 64 bits).
+I6_ROW_FN bool strip_rows_taken(const bool best_path, const long long T, const long long SP) { return best_path || strip_rows_fit(T, SP); }

@@ -11,7 +11,7 @@ PROGRAM = r"""
 #include "strip_rows.h"
 #include <cstdio>
 #include <cstdlib>
-// fits, lowest offset of a lane without a state, highest of one with a state, end of the rows, for L = T
+// taken in the full sum, in the best path, lowest offset of a lane without a state, highest of one with a state, end of the rows, for L = T
 int main(int argc, char** argv) {
     for (int i = 1; i + 1 < argc; i += 2) {
         const int T = atoi(argv[i]), SP = atoi(argv[i + 1]);
@@ -21,7 +21,7 @@ int main(int argc, char** argv) {
             low = none < low ? none : low;
             if (t < T) high = last > high ? last : high;
         }
-        printf("%d %u %u %lld\n", (int)strip_rows_fit(T, SP), low, high, 4LL * T * SP);
+        printf("%d %d %u %u %lld\n", (int)strip_rows_taken(false, T, SP), (int)strip_rows_taken(true, T, SP), low, high, 4LL * T * SP);
     }
     return 0;
 }
@@ -47,10 +47,11 @@ def test_rows_at_the_limit(rows, SP):
     if SP >= 1552:                              # (every row is walked over)
         sizes += [(345921, 1552), (133681, 4016), (131586, 4080)]
     got = rows(sizes)
-    for (T, sp), (fits, low, high, end) in zip(sizes, got):
+    for (T, sp), (fits, path, low, high, end) in zip(sizes, got):
         assert bool(fits) == (4 * -(-T // 8) * 8 * sp < 2 ** 31)
+        assert path                             # (stores no such rows)
         if fits:
             assert high == end - 4              # the last state of the last row is the last word
             assert low >= end                   # and a lane without a state is never in front of it
-    wrapped = [low < end for (_, low, _, end) in got]
+    wrapped = [low < end for (_, _, low, _, end) in got]
     assert SP < 1552 or any(wrapped)            # (there are such sizes)

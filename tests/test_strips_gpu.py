@@ -108,6 +108,22 @@ def test_best_path_over_many_chunks(oracle):
         assert_identical(run_cabi_viterbi(*args)[:2], oracle.viterbi_oracle(*args))
 
 
+def test_best_path_beyond_the_rows_of_the_full_sum(oracle):
+    """131100 frames of 4090 states: more than 2 GiB of the rows that only the full sum stores, so no reason to leave the strips out.  (That they
+    are there is seen from a wait that runs out: the search that would take their place has none.)"""
+    rng = np.random.default_rng(42)
+    edges, weights, start_end, n = automata(rng, [4090], 8, "chain")
+    am = rng.normal(size=(131100, 1, 8)).astype(np.float32)
+    args = (am, edges, weights, start_end, np.array([131093], dtype=np.int32), n)
+    assert_identical(run_cabi_viterbi(*args)[:2], oracle.viterbi_oracle(*args))
+    cabi.set_spin_limit(1)
+    try:
+        _, scores, code = run_cabi_viterbi(*args, check=False)
+    finally:
+        cabi.set_spin_limit(0)
+    assert code == -15 and np.isnan(scores[0])
+
+
 @pytest.mark.parametrize("B", [1, 8])
 @pytest.mark.parametrize("n_frames", [9, 16, 23, 50, 64, 127, 200, 249, 256])
 def test_best_path_of_short_ctc_automata(oracle, n_frames, B):
