@@ -259,11 +259,12 @@ __device__ inline bool strip_shape(const int S, const int n_edges, const int edg
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
     return vit_strip_bytes(n, T8, T, round16(S)) <= 4LL * T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
 }
-// The rows of the best path (64 floats per strip and frame) stand behind the score of a state in the strips' score table, or in beta's area
-// where every edge has a score of its own.
+// The rows of the best path (64 floats per strip and frame) stand behind the scores in the strips' score table, or, for several strips in which
+// every edge has a score of its own, in beta's area.  (The table has room for three scores and the row of a lane of one strip, 256 of its 272 floats a
+// sequence; beta's share of an automaton of a handful of edges is smaller than a row.)
 __device__ inline bool vit_rows_fit(const int S, const int n_edges, const int edge_begin, const int b, const int T, const int emit) {
     const long long T8 = (T + STRIP_FRAMES - 1) / STRIP_FRAMES * STRIP_FRAMES;
-    return emit != EMIT_EDGE || 64LL * strips_of(S) * T8 <= T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
+    return emit != EMIT_EDGE || strips_of(S) == 1 || 64LL * strips_of(S) * T8 <= T * (state_off(edge_begin + n_edges, b + 1) - state_off(edge_begin, b));
 }
 // A batch goes through the strips as a whole or not at all: with some of its sequences left to the other recursion (or search),
 // which then runs behind the strips, a call took as long as both (8 sequences of 510-690 states, some of them on the other

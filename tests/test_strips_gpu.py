@@ -23,7 +23,8 @@ def automata(rng, sizes, F, kind, permute=False):
     passed over; "ctc" emission on the target state and several edges into the last state; "wide" edges of up to four
     states upward, some of them twice; "far" one edge of five (not for the strips); "mixed" that in the last sequence only;
     "sparse" like wide, but few of those edges, and "passing" like optional, but few such states (2.05 and 2.3 edges per state at
-    most, what the full sum leaves to the strips).  Weights are multiples of 1/2, so ties are common."""
+    most, what the full sum leaves to the strips); "own" and "own skip" like chain and passing, but every edge has an emission of
+    its own, with "end" an end state that no edge leaves, entered by five edges from up to four states below.  Weights are multiples of 1/2, so ties are common."""
     frm, to, emis, seq, w = [], [], [], [], []
     ends = []
     off = 0
@@ -41,6 +42,8 @@ def automata(rng, sizes, F, kind, permute=False):
                 steps.append(2)
             if kind == "passing" and rng.random() < 0.2:
                 steps.append(2)
+            if kind.startswith("own skip") and rng.random() < (0.2 if n > 600 else 0.01):
+                steps.append(2)
             if kind == "sparse" and (u % 60 in (1, 56, 57) or u in (235, 236, 239)) and (u // 60) % 2 == 0:
                 steps.append(int(rng.choice([1, 3, 4, 2])))
             if kind == "wide":
@@ -48,11 +51,14 @@ def automata(rng, sizes, F, kind, permute=False):
             if (kind == "far" or (kind == "mixed" and b == len(sizes) - 1)) and u == n // 3:
                 steps.append(5)
             for k in steps:
-                if u + k < n and not (kind == "ctc" and u + k == n - 1 and k == 0):
-                    edge(u, u + k, state_emis[u + k] if by_target else state_emis[u])
+                if u + k < n and not (kind.endswith(("ctc", "end")) and u + k == n - 1 and k == 0):
+                    edge(u, u + k, rng.integers(0, F) if kind.startswith("own") else state_emis[u + k] if by_target else state_emis[u])
         if kind == "ctc" and n >= 5:
             for u, v in ((n - 2, n - 2), (n - 3, n - 2), (n - 4, n - 2), (n - 2, n - 3)):
                 edge(u, n - 1, state_emis[v])
+        if kind.endswith("end") and n >= 5:
+            for u in (n - 2, n - 3, n - 4, n - 5):
+                edge(u, n - 1, rng.integers(0, F))
         ends.append(off + n - 1)
         off += n
     starts = np.concatenate([[0], np.cumsum(sizes)[:-1]])
@@ -94,6 +100,30 @@ def test_best_path(oracle, case, permute):
     args = (am, edges, weights, start_end, seq_lens, n)
     align, scores, _ = run_cabi_viterbi(*args)
     assert_identical((align, scores), oracle.viterbi_oracle(*args))
+
+
+OWN = ["own", "own skip", "own end", "own skip end"]
+
+
+@pytest.mark.parametrize("kind", OWN)
+@pytest.mark.parametrize("sizes,T", [([61, 125, 180, 301, 59], 420), ([60, 121, 241, 5], 256), ([900, 640, 1201], 1300)])
+def test_best_path_with_a_score_per_edge(oracle, kind, sizes, T):
+    """No state has one score: a score per class of edge in the strips' table, two or three classes; with and without an end state whose edges are
+    left out of its strip; one strip and many, short sequences and chunks."""
+    rng = np.random.default_rng(len(kind) + T)
+    edges, weights, start_end, n = automata(rng, sizes, 300, kind, permute=T == 420)
+    lens = np.array([T - k for k in (0, 7, 2, 5, 4)[:len(sizes)]], dtype=np.int32)
+    for am in (rng.normal(size=(T, len(sizes), 300)).astype(np.float32), -0.25 * rng.integers(0, 12, size=(T, len(sizes), 300)).astype(np.float32)):
+        args = (am, edges, weights, start_end, lens, n)
+        want = oracle.viterbi_oracle(*args)
+        assert_identical(run_cabi_viterbi(*args)[:2], want)
+    assert np.isfinite(want[1]).all()
+    if max(sizes) > 240:        # (a wait between workgroups that runs out, which only the strips have: they were there)
+        cabi.set_spin_limit(1)
+        try:
+            assert run_cabi_viterbi(*args, check=False)[2] == -15
+        finally:
+            cabi.set_spin_limit(0)
 
 
 def test_best_path_over_many_chunks(oracle):
