@@ -180,6 +180,26 @@ def test_best_path_of_short_ctc_automata(oracle, n_frames, B):
         assert_identical(got[:2], oracle.viterbi_oracle(am, edges[:, there].copy(), weights[there].copy(), start_end, lens, int(n)))
 
 
+@pytest.mark.parametrize("n_frames", [257, 320, 321, 385])
+def test_best_path_of_ctc_automata_that_end_with_a_chunk(oracle, n_frames):
+    """Chunks of 64 frames: sequences that end with one, with the first frame of the next, and all around that."""
+    from i6_native_ops_amd.fsa import ctc_fsa
+    rng = np.random.default_rng(n_frames)
+    F = 29
+    lens = np.array([max(1, n_frames - d) for d in (0, 1, 2, 7, 8, 63, 64, 65, 66, 128, 129, 250)], dtype=np.int32)
+    n_labels = np.array([rng.integers(1, max(2, n // 2)) for n in lens], dtype=np.int32)
+    targets = rng.integers(1, F, size=(lens.size, int(n_labels.max()))).astype(np.int32)
+    n, edges, weights, start_end = (x.cpu().numpy() if torch.is_tensor(x) else x for x in
+                                    ctc_fsa(torch.from_numpy(targets).cuda(), torch.from_numpy(n_labels).cuda()))
+    there = edges[3] >= 0
+    for rep in range(2):
+        am = rng.normal(size=(n_frames, lens.size, F)).astype(np.float32)
+        if rep == 1:
+            am = np.round(2 * am) / 4
+        got = run_cabi_viterbi(am, edges, weights, start_end, lens, int(n))
+        assert_identical(got[:2], oracle.viterbi_oracle(am, edges[:, there].copy(), weights[there].copy(), start_end, lens, int(n)))
+
+
 def test_scores_that_are_not_numbers():
     """A NaN never wins, -inf closes an edge, a class of +inf takes everything: as in the other kernels (the reference's
     compare-and-swap does something else with a NaN)."""
@@ -278,6 +298,15 @@ def test_full_sum(oracle, case, permute):
     check_full_sum(oracle, args, strips=not (permute and case in (0, 1, 4)))
 
 
+@pytest.mark.parametrize("kind", OWN)
+@pytest.mark.parametrize("sizes,T", [([177, 180, 240, 296], 312), ([700, 650, 1201], 1288)])
+def test_full_sum_with_a_score_per_edge(oracle, kind, sizes, T):
+    rng = np.random.default_rng(len(kind) + T)
+    edges, weights, start_end, n = automata(rng, sizes, 300, kind)
+    am = rng.uniform(0.1, 9.0, size=(T, len(sizes), 300)).astype(np.float32)
+    check_full_sum(oracle, (am, edges, -weights, start_end, np.array([T - k for k in (0, 7, 2, 5)[:len(sizes)]], dtype=np.int32), n))
+
+
 @pytest.mark.parametrize("n_frames", [257, 258, 263, 264])
 def test_full_sum_last_state_alone_in_a_strip(oracle, n_frames):
     """Backward strips hold the states from 60 j - 4 on: with 57 states more than a multiple of 60 the end state has the last one to
@@ -290,8 +319,8 @@ def test_full_sum_last_state_alone_in_a_strip(oracle, n_frames):
 
 @pytest.mark.parametrize("labels", [(27, 30, 28, 29), (57, 58, 87, 60), (119, 147, 118, 120), (260, 300, 297, 290)])
 def test_full_sum_ctc(oracle, labels):
-    """CTC automata as ctc_fsa leaves them (arrays at their capacity): an end state with five entering edges, alone in a strip or beside others, and
-    last frames everywhere in a block; a repeated label at the end."""
+    """CTC automata as ctc_fsa leaves them (arrays at their capacity): an end state with five entering edges, alone in a strip or beside others; a
+    repeated label at the end."""
     from i6_native_ops_amd.fsa import ctc_fsa
     from tests.gpu_util import DeviceProblem
     from tests.helpers import posterior
@@ -303,6 +332,30 @@ def test_full_sum_ctc(oracle, labels):
     am = rng.uniform(0.1, 9.0, size=(T, 4, F)).astype(np.float32)
     n, edges, weights, start_end = (x.cpu().numpy() if torch.is_tensor(x) else x for x in
                                     ctc_fsa(torch.from_numpy(targets).cuda(), torch.from_numpy(np.array(labels, dtype=np.int32)).cuda()))
+    there = edges[3] >= 0
+    want_out, want_loss = oracle.fbw_oracle(am, edges[:, there].copy(), weights[there].copy(), start_end, lens, int(n), threads=4)
+    P = DeviceProblem(am, edges, weights, start_end, lens, n)
+    strips = P.run(cabi.OUT_PROB)[0].cpu().numpy()
+    np.testing.assert_allclose(P.loss.cpu().numpy(), want_loss, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(strips, posterior(want_out), rtol=0, atol=1e-4)
+    P.ws_bytes -= 256       # without the strips' tables: other bits show that they were there
+    assert not np.array_equal(strips, P.run(cabi.OUT_PROB)[0].cpu().numpy())
+
+
+@pytest.mark.parametrize("label", [28, 59, 147])
+def test_full_sum_ctc_last_frames(oracle, label):
+    """Last frames everywhere in a block: beta leaves the end state there, in the first block of its walk or into the next one."""
+    from i6_native_ops_amd.fsa import ctc_fsa
+    from tests.gpu_util import DeviceProblem
+    from tests.helpers import posterior
+    rng = np.random.default_rng(label)
+    B, F, T = 9, 23, max(272, 5 * label // 2)
+    lens = np.array([T - b for b in range(B)], dtype=np.int32)
+    targets = rng.integers(1, F, size=(B, label + 1)).astype(np.int32)
+    targets[1::3, label - 1] = targets[1::3, label - 2]
+    n_labels = np.array([label + (b % 2) for b in range(B)], dtype=np.int32)
+    am = rng.uniform(0.1, 9.0, size=(T, B, F)).astype(np.float32)
+    n, edges, weights, start_end = (x.cpu().numpy() if torch.is_tensor(x) else x for x in ctc_fsa(torch.from_numpy(targets).cuda(), torch.from_numpy(n_labels).cuda()))
     there = edges[3] >= 0
     want_out, want_loss = oracle.fbw_oracle(am, edges[:, there].copy(), weights[there].copy(), start_end, lens, int(n), threads=4)
     P = DeviceProblem(am, edges, weights, start_end, lens, n)
