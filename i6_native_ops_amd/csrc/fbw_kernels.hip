@@ -354,6 +354,11 @@ inline int strip_density(const int T, const int B, const int E, const int n_stat
         // without (a workgroup per sequence, three to six candidates per state; what the strips cost is 190 ns a frame): 64 sequences of 200-600 states, T=1203: 810 / 942
         // us (recursion 540 -> 250); 1 of 400 and 630, T=2302 and 3576: 486 / 1162, 699 / 1950; 10 of 1200, T=3746: 1661 / 3103; 59 of 260, T=516: 251 / 315; 16 of
         // 80, T=300 F=50000: 289 / 311.
+        // On both sides of the line: 81 states, T=300 F=500, B=32 132 / 157, 64 155 / 174, 96 175 / 192, 128 194 / 212, 256 317 / 297; 201 states, T=500, B=64 230 / 269,
+        // 96 287 / 318, 128 333 / 349, 256 573 / 547; 401 states, T=900, B=64 420 / 546, 96 644 / 671, 128 742 / 753; 901 states, T=2000, B=32 1292 / 2095, 38 1563 /
+        // 2175: the two cross behind it, at 1.3 to 4 times as many workgroups.
+        // A batch of that density which the preparation leaves to the other recursion pays for the preparation's fourth role and for fbw_strips, which finds nothing to
+        // do: 180 states of 2.7 edges (some of three states upward), T=500 F=264, B=8 157 -> 161, 32 180 -> 185; 90 states, T=300 B=60 141 -> 147.
         const long long states = std::min(strip_states(B, E), (long long)n_states / B + 1), n = 2LL * B * strip_groups(states);
         return n <= (states > 256 ? 3 * n_cu / 2 : n_cu / 2) ? 310 : 0;
     }
@@ -364,10 +369,10 @@ inline int strip_density(const int T, const int B, const int E, const int n_stat
 }
 // Best path: the same question.  Call with strips / without: chains and 2.14 edges per state, 60-180 states 0.62 ... 0.95 and 0.99 at n=256;
 // 375 states 0.60 ... 0.86 at n=256, 0.99 at 384, 1.11 at 512; 900 states 0.43 ... 0.70 at 768; 1750 states 0.27 ... 0.87 at 768, 1.16
-// at 1024.  More than 2.4 edges per state (measured with edges of any kind in CTC's last strip, which it no longer has): 81 states
-// 0.95 up to n=64, 1.02 at 96, 1.07 at 128; 201 and 401 states 0.77 ... 0.86-0.99 at 64, 1.02-1.05 at 128; 551-851 states 0.50 ... 0.80 at 256,
-// 1.02 at 384; 1001 states 0.46 ... 0.53 at 1280 (more than 1024 states of that degree: 3.4 us a frame in the search);
-// five edges per state, 375 states: 0.95 up to 32, 1.01 at 64, 1.5 beyond 256; and slower than the search beside the gather (1.09).
+// at 1024.  More than 2.4 edges per state: in CTC automata a state has one score and the strips are fast: 81 states 0.51 at n=32, 0.58 at 64, 0.62 at 128, 0.69 at 256
+// (T=300); 201 states 0.47 at 32, 0.55 at 64, 0.68 at 128, 0.84 at 256 (T=500); 401 states 0.35 at 32, 0.41 at 64, 0.51 at 128, 0.70 at 192, 0.84 at 256 (T=900); 901 states
+// 0.18 at 32 ... 0.41 at 152 (T=2000).  With edges of any kind in every strip, which the host cannot tell from those (five edges per state, 375 states), 0.95 up to 32, 1.01 at
+// 64, 1.5 beyond 256: the line is where these cross.  And slower than the search beside the gather (1.09).
 inline bool best_path_strips(const int B, const int E, const int n_states, const int n_cu, const bool overlap) {
     const long long states = std::min((long long)n_states, (long long)E + B) / B + 1, n = B * strip_groups(states);
     if (10LL * E > 24LL * n_states) return !overlap && n <= (states > 1024 ? 4LL * n_cu : states > 512 ? n_cu : n_cu / 4);
@@ -497,7 +502,7 @@ struct PrepArgs {
     int strips = 0;         // > 0: a batch of sequences of up to that many strips goes to the strip kernels ...
     int strip_density = 0;  // ... if none has more than this many edges per 100 states (0: any number)
     int level = 0;          // 1: every sequence whose ids do not follow the automaton gets numbers along it; 2: those of at most strip_density edges per 100 states
-    unsigned short* sslot = nullptr;   // per state: slot of its score, where it has one (STRIP_EMIT)
+    unsigned short* sslot = nullptr;   // per state: slot of its score, where it has one (EMIT_MASK)
     int* sprog = nullptr;   // their progress counters, 2 * STRIP_MAX per sequence; the last one is the mark of strip_lost
     int roles() const { return strips > 0 && !best_path ? 4 : 3; }      // workgroups per sequence
 };
@@ -738,7 +743,7 @@ __device__ __forceinline__ void prepare_sequence(const PrepArgs& a, unsigned* ld
     // count): the states get dense numbers (below), and the sequence takes the general path, which
     // looks them up
     const bool sparse = !err && n_edges > 0 && S > 2LL * n_edges + 2;
-    // up to this many edges the renumbering is done in LDS, the same way by all three roles, and the
+    // up to this many edges the renumbering is done in LDS, the same way by all roles, and the
     // sequence stays on the fast kernels: the 2n+2 ids fit the key array, and afterwards the n edge
     // keys its lower half and the distinct ids its upper half
     constexpr int RENUM_LDS_EDGES = EB_MAX / 2 - 1;

@@ -126,6 +126,38 @@ def test_best_path_with_a_score_per_edge(oracle, kind, sizes, T):
             cabi.set_spin_limit(0)
 
 
+# sequences, frames, states from .. to, kind: what follows the paths is a matter of these (best_path_walk)
+WALKS = [
+    (100, 300, 60, 160, "chain"),           # one workgroup a sequence
+    (64, 512, 66, 70, "own end"),           # the same, in pieces, with bytes
+    (60, 449, 40, 80, "ctc"),               # with an end state looked up apart
+    (2, 500, 10, 30, "ctc"),
+    (3, 130, 125, 200, "optional"),         # few frames of many states: chunks in the search's kernel
+    (100, 520, 60, 120, "optional"),        # a kernel of their own
+    (60, 450, 100, 200, "ctc"),
+    (60, 450, 100, 200, "own skip end"),
+    (60, 600, 290, 300, "chain"),
+]
+
+
+@pytest.mark.parametrize("case", range(len(WALKS)))
+def test_best_path_whoever_follows_it(oracle, case):
+    B, T, lo, hi, kind = WALKS[case]
+    rng = np.random.default_rng(600 + case)
+    edges, weights, start_end, n = automata(rng, rng.integers(lo, hi + 1, size=B).tolist(), 50, kind)
+    lens = rng.integers(max(hi, T // 2), T + 1, size=B).astype(np.int32) if hi < T // 2 else rng.integers(T - 9, T + 1, size=B).astype(np.int32)
+    for am in (rng.normal(size=(T, B, 50)).astype(np.float32), -0.25 * rng.integers(0, 12, size=(T, B, 50)).astype(np.float32)):
+        args = (am, edges, weights, start_end, lens, n)
+        assert_identical(run_cabi_viterbi(*args)[:2], oracle.viterbi_oracle(*args))
+    if lo > 240:        # a wait between workgroups that runs out: no path and no score (and the strips were there)
+        cabi.set_spin_limit(1)
+        try:
+            align, scores, code = run_cabi_viterbi(*args, check=False)
+        finally:
+            cabi.set_spin_limit(0)
+        assert code == -15 and np.isnan(scores).all() and not align.any()
+
+
 def test_best_path_over_many_chunks(oracle):
     """Where the paths lead over a chunk of 64 frames is written by one workgroup and read by another, in the same kernel and, for most numbers of states,
     from cache lines that several have written: other scores in the same workspace, again and again."""
