@@ -178,7 +178,11 @@ def test_degree_just_beyond_the_register_tables(oracle, n_mid):
                           rng.integers(0, W.F, size=2 * n_mid), [b] * (2 * n_mid)], dtype=np.int32)
         edges = np.concatenate([edges, extra], axis=1)
         weights = np.concatenate([weights, rng.uniform(0.2, 2.0, size=2 * n_mid).astype(np.float32)])
-    check_against_oracle(oracle, (W.am_scores, edges, weights, W.start_end_states, W.seq_lens, W.n_states), bitwise=n_mid <= 15 - 3)
+    # (with 12 extra edges a state of the third sequence, which is drawn as a target as well, comes to 16 leaving edges: the general path, whose atomics
+    # add up in no fixed order -- a posterior of 1.5e-36 has differed by its last bit)
+    degree = max(int(np.bincount(ids[edges[3] == b]).max()) for ids in edges[:2] for b in range(W.B))
+    assert n_mid > 9 or degree <= 15
+    check_against_oracle(oracle, (W.am_scores, edges, weights, W.start_end_states, W.seq_lens, W.n_states), bitwise=n_mid <= 15 - 3 and degree <= 15)
     e2, w2, s2, t2, n2 = fan(rng, 12, 9, n_mid)
     am = rng.uniform(0.1, 3.0, size=(12, 1, 9)).astype(np.float32)
     check_against_oracle(oracle, (am, e2, w2, np.array([[s2], [t2]], np.int32), np.array([12], np.int32), n2), bitwise=n_mid <= 15)
