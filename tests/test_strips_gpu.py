@@ -189,7 +189,7 @@ def test_best_path_beyond_the_rows_of_the_full_sum(oracle):
 @pytest.mark.parametrize("B", [1, 8])
 @pytest.mark.parametrize("n_frames", [9, 16, 23, 50, 64, 127, 200, 249, 256])
 def test_best_path_of_short_ctc_automata(oracle, n_frames, B):
-    """Up to 256 frames one workgroup follows the path as a whole, from an end state whose edges are looked up apart from the others': last frames
+    """Few frames of few states: one workgroup follows the path as a whole (chunks where there are more), from an end state whose edges are looked up apart from the others': last frames
     everywhere in a block, short sequences behind long ones, repeated labels at the end, scores with and without ties."""
     from i6_native_ops_amd.fsa import ctc_fsa
     rng = np.random.default_rng(10 * n_frames + B)
